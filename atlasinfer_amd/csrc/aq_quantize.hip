@@ -600,8 +600,8 @@ __device__ __forceinline__ uint32_t quot2(uint32_t xp, float r) {
   return q;
 }
 
-// Code exchange of a workgroup of four 4096-element rows (per-channel
-// blocks): 16-byte piece (column piece c, row r) at slot 4 c + r, the low
+// Code exchange of a workgroup of four rows of 2049 to 4096 elements
+// (per-channel blocks): 16-byte piece (column piece c, row r) at slot 4 c + r, the low
 // four bits XORed with bits 4-7 so that both the writes (lanes 16 slots
 // apart) and the reads (consecutive slots) spread over the LDS banks.
 __device__ __forceinline__ int xchg_slot(int i) { return i ^ ((i >> 4) & 15); }
@@ -828,6 +828,7 @@ __device__ __forceinline__ void finish_block_fast(const QuantArgs& a, Elems<E>& 
 #pragma unroll
     for (int i = 0; i < E / 16; i++) {
       const int c = (threadIdx.x >> 2) + i * 64;
+      if (MODE != kFullBlocks && c >= (int)(G >> 4)) break;  // rows of fewer than 4096 have fewer column pieces
       *reinterpret_cast<uint4*>(a.codes + tiled_offset(row0 + rr, (int64_t)c << 4, a.nchunks)) =
           xchg[xchg_slot((c << 2) | rr)];
     }
@@ -907,7 +908,7 @@ __global__ __launch_bounds__(TAU > kWG ? TAU : kWG) void quantize_kernel(QuantGr
     finish_block_any<TAU, E, MODE>(a, xs, g, gvalid, base, i0, t, lds_d + team * NWT, lds_f + team * NWT,
                                    lds_i + 2 * team * NWT);
   else {
-    // four one-row blocks of 4096 elements staged together, tiled codes:
+    // four one-row blocks of 2049 to 4096 elements staged together, tiled codes:
     // the codes go out through the stage in 64-byte runs (a store
     // instruction of 16-byte pieces, one per lane, would otherwise touch 64
     // cache lines)

@@ -132,6 +132,33 @@ def test_quantize_matches_oracle(oracle, rows, cols, G, thr, fmt, tdof, frac):
     assert np.array_equal(bits(deq), bits(oracle.dequantize(ref)))
 
 
+@pytest.mark.parametrize("rows,cols", [(48, 2176), (32, 2304), (16, 3584), (64, 3968)])
+def test_short_rows_keep_their_codes_inside(oracle, rows, cols):
+    """Per-channel rows of 2049 to 4095 elements into tiled codes: the
+    four-row code exchange of a workgroup writes the row's own column pieces
+    only (it wrote 4096 elements' worth, into the next tile row and past the
+    end), so every code is the oracle's and the bytes after a C caller's code
+    buffer stay as they were."""
+    rng = np.random.default_rng(rows + cols)
+    w = make_weights(rng, (rows, cols), t_dof=3, frac=0.01)
+    ref = oracle.quantize(w, cols, 3.0, oracle.FMT_E4M3)
+    x = torch.from_numpy(w).to(DEV)
+    L = _lib.load()
+    guard = 1 << 16
+    codes = torch.full((rows * cols + guard,), 0xA5, dtype=torch.uint8, device=DEV)
+    scales = torch.empty(rows, dtype=torch.float16, device=DEV)
+    off = torch.empty(rows + 1, dtype=torch.int32, device=DEV)
+    ws = torch.empty(int(L.aq_quantize_workspace_size(rows * cols, cols)), dtype=torch.uint8, device=DEV)
+    thr = int(np.float16(3.0).view(np.uint16))
+    _lib.check(L.aq_quantize(x.data_ptr(), rows * cols, cols, thr, _lib.FMT_E4M3, cols, _lib.LAYOUT_TILED,
+                             codes.data_ptr(), scales.data_ptr(), off.data_ptr(), ws.data_ptr(), ws.numel(),
+                             _lib.stream_of(x.device)), "aq_quantize")
+    got = codes.cpu().numpy()
+    assert np.array_equal(got[: rows * cols], tile_np(ref["codes"], rows, cols))
+    assert (got[rows * cols:] == 0xA5).all()
+    assert np.array_equal(bits(scales), bits(ref["scale_factors"]))
+
+
 def test_llama_shape_per_channel_e4m3_full(oracle):
     """A full 4096 x 4096 projection at the product setting (per-channel e4m3)."""
     rng = np.random.default_rng(5)
