@@ -53,6 +53,7 @@ SIGNATURES = {
     "aq_tile_codes": (ctypes.c_int, [_P, _I64, _I64, _P, _P]),
     "aq_untile_codes": (ctypes.c_int, [_P, _I64, _I64, _P, _P]),
     "aq_dequantize": (ctypes.c_int, [_P, _P, _I64, _I64, ctypes.c_int, _I64, ctypes.c_int, _P, _P, _I64, _P, _P]),
+    "aq_dequantize_stream": (ctypes.c_int, [_P, _P, _I64, _I64, _P, _P, _I64, _P, _P]),
     "aq_zscore": (ctypes.c_int, [_P, _I64, ctypes.c_float, _P, _P, _P]),
     "aq_qlinear_workspace_size": (_I64, [_I64, _I64, _I64]),
     "aq_qlinear": (ctypes.c_int, [_P, _I64, _I64, _I64, _P, _P, _I64, ctypes.c_int, _I32P, _I32P, _P, _I32P, _P,

@@ -710,14 +710,19 @@ def dequantize_tensor(quant_data: QuantizedTensor, target_device: torch.device) 
         dev = _lib.compute_device(target_device)
         q = quant_data.to(dev)
         fmt = _format_id(q.code_format)
-        codes = _stored_codes(q, dev)
         _, K = _rows_cols(q.original_shape)
         out = torch.empty(numel, dtype=torch.float16, device=dev)
         nnz = q.outlier_indices.numel()
-        _lib.check(L.aq_dequantize(codes.data_ptr(), q.scale_factors.data_ptr(), numel, q.block_size, fmt, K,
-                                   _lib.LAYOUTS[q.code_layout], _lib.ptr(q.outlier_indices),
-                                   _lib.ptr(q.fp16_outliers), nnz, out.data_ptr(), _lib.stream_of(dev)),
-                   "aq_dequantize")
+        if q.code_format == "int8" and q.code_layout == "flat":  # straight from the compacted stream
+            _lib.check(L.aq_dequantize_stream(_lib.ptr(q.fp8_data), q.scale_factors.data_ptr(), numel, q.block_size,
+                                              _lib.ptr(q.outlier_indices), _lib.ptr(q.fp16_outliers), nnz,
+                                              out.data_ptr(), _lib.stream_of(dev)), "aq_dequantize_stream")
+        else:
+            codes = _stored_codes(q, dev)
+            _lib.check(L.aq_dequantize(codes.data_ptr(), q.scale_factors.data_ptr(), numel, q.block_size, fmt, K,
+                                       _lib.LAYOUTS[q.code_layout], _lib.ptr(q.outlier_indices),
+                                       _lib.ptr(q.fp16_outliers), nnz, out.data_ptr(), _lib.stream_of(dev)),
+                       "aq_dequantize")
         final = out.view(q.original_shape).to(target_device)
 
     with _cache_lock:

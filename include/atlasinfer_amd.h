@@ -210,6 +210,16 @@ int aq_dequantize(const void* codes, const void* scales, int64_t numel, int64_t 
                   const int64_t* flat_idx, const void* vals, int64_t nnz, void* out, void* stream);
 
 /*
+ * aq_expand_codes followed by aq_dequantize of a weight in the reference's
+ * compacted int8 form, in one pass: stream_codes int8 [padded - nnz] as
+ * aq_compact_codes writes them, flat_idx ascending.  Bit for bit the result
+ * of the two calls.  Serves dequantize_tensor (adaptive_quantizer.py:185-245)
+ * for tensors kept in that form.
+ */
+int aq_dequantize_stream(const void* stream_codes, const void* scales, int64_t numel, int64_t G,
+                         const int64_t* flat_idx, const void* vals, int64_t nnz, void* out, void* stream);
+
+/*
  * calculate_zscore_manual (adaptive_quantizer.py:44-49) of x[n] as one
  * block: z = fp16(fp16(x - mean) / fp16(std + eps)).  stats (may be NULL)
  * receives (mean, std, std + eps) as fp16.  n <= aq_max_block_size().
