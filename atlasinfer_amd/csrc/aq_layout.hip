@@ -406,7 +406,44 @@ __global__ __launch_bounds__(256) void outlier_tile_rows_kernel(const int32_t* r
   for (int r = 0; r <= 16; r++) src.rs[r] = row_ptr[(int64_t)(rb * 16 + r) * rstride];
   src.cols = cols;
   src.vals = vals;
-  aq::tile_row_sort<256>(src, rb, nch, src.rs[0], src.rs[16], sm, part, tile_ptr, tile_ent, tile_max);
+  aq::tile_row_sort<256, 4>(src, rb, nch, src.rs[0], src.rs[16], sm, part, tile_ptr, tile_ent, tile_max);
+}
+
+constexpr int kTileMaxWG = 32;  // workgroups a list
+__global__ __launch_bounds__(256) void tile_max_kernel(aq::TileMaxGroup g) {
+  __shared__ int part[4];
+  const int m = blockIdx.x / kTileMaxWG;
+  const int32_t* p = nullptr;
+  int32_t* out = nullptr;
+  int64_t n = 0;
+#pragma unroll
+  for (int j = 0; j < aq::kMaxTileMax; j++)
+    if (j == m) {
+      p = g.tile_ptr[j];
+      n = g.n[j];
+      out = g.tile_max[j];
+    }
+  if (!out) return;
+  int mx = 0;
+  // eight blocks a thread and round, their loads in flight together
+  for (int64_t i0 = (int64_t)(blockIdx.x % kTileMaxWG) * 2048 + threadIdx.x; i0 < n; i0 += 2048 * kTileMaxWG) {
+    int lo[8], hi[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      const int64_t i = min(i0 + 256 * k, n - 1);
+      lo[k] = p[i];
+      hi[k] = p[i + 1];
+    }
+#pragma unroll
+    for (int k = 0; k < 8; k++) mx = max(mx, hi[k] - lo[k]);
+  }
+  for (int d = 32; d >= 1; d >>= 1) mx = max(mx, __shfl_xor(mx, d));
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = mx;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    mx = max(max(part[0], part[1]), max(part[2], part[3]));
+    if (mx > 0) raise_to(out, mx);
+  }
 }
 
 // One thread per block of 16 rows x 64 columns (tile row rb, chunk c), for
@@ -603,17 +640,30 @@ extern "C" int aq_dequantize_stream(const void* stream_codes, const void* scales
   return AQ_OK;
 }
 
+hipError_t aq::launch_tile_max(const TileMaxGroup& g, int count, hipStream_t stream) {
+  hipLaunchKernelGGL(tile_max_kernel, dim3((unsigned)(count * kTileMaxWG)), dim3(256), 0, stream, g);
+  return hipGetLastError();
+}
+
 hipError_t aq::launch_outlier_tiles(const int32_t* row_ptr, int64_t rstride, const int32_t* cols, const uint16_t* vals,
-                                   int64_t N, int64_t K, int32_t* tile_ptr, uint32_t* tile_ent, int32_t* tile_max,
-                                   hipStream_t stream) {
+                                    int64_t N, int64_t K, int32_t* tile_ptr, uint32_t* tile_ent, int32_t* tile_max,
+                                    hipStream_t stream) {
   const int64_t nblk = (N / 16) * (K / 64);
-  if (K / 64 <= aq::kTileRowsMaxChunks)
+  if (K / 64 <= aq::kTileRowsMaxChunks) {
+    const bool raise = N / 16 <= aq::kRaiseTileRows;
     hipLaunchKernelGGL(outlier_tile_rows_kernel, dim3((unsigned)(N / 16 + 1)), dim3(256),
                        (size_t)33 * (K / 64) * sizeof(int), stream, row_ptr, rstride, cols, vals, (int)(N / 16),
-                       (int)(K / 64), tile_ptr, tile_ent, tile_max);
-  else
-    hipLaunchKernelGGL(outlier_tiles_kernel, dim3((unsigned)aq::ceil_div(nblk + 1, 256)), dim3(256), 0, stream,
-                       row_ptr, rstride, cols, vals, (int)(N / 16), (int)(K / 64), tile_ptr, tile_ent, tile_max);
+                       (int)(K / 64), tile_ptr, tile_ent, raise ? tile_max : nullptr);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || !tile_max || raise) return e;
+    TileMaxGroup g{};
+    g.tile_ptr[0] = tile_ptr;
+    g.n[0] = nblk;
+    g.tile_max[0] = tile_max;
+    return launch_tile_max(g, 1, stream);
+  }
+  hipLaunchKernelGGL(outlier_tiles_kernel, dim3((unsigned)aq::ceil_div(nblk + 1, 256)), dim3(256), 0, stream, row_ptr,
+                     rstride, cols, vals, (int)(N / 16), (int)(K / 64), tile_ptr, tile_ent, tile_max);
   return hipGetLastError();
 }
 

@@ -24,9 +24,11 @@
 //          equals the round-to-nearest-even encoding on every fp16 in
 //          [-448, 448])
 // Outliers are compacted inside the team with a prefix sum (shuffles + LDS)
-// into a per-block staging slot; a scan over the per-block counts and a
+// into a staging slot per wave; a scan over the per-block counts and a
 // gather pass then write the ascending outlier list.
 #include <math.h>
+
+#include <algorithm>
 
 #include "aq_common.h"
 #include "aq_tiles.h"
@@ -53,14 +55,32 @@ struct QuantArgs {
   int64_t K;        // row length for the tiled layout
   int64_t nchunks;  // K / 128
   int64_t bpr;      // tiled layout: blocks per row, K / G
+  int bshift;       // log2(bpr) when it is a power of two, else -1
   double inv_g;     // RN64(1 / G)
   float inv_g1;     // RN32(1 / (G - 1)) (G >= 2)
   uint8_t* codes;
   uint16_t* scales;
   int32_t* block_cnt;  // block_off, holds counts until the scan
-  int32_t* stage_col;
-  uint16_t* stage_val;
+  uint32_t* stage;     // outliers by staging unit (unit_blocks)
 };
+
+// Outliers are staged by unit: the blocks of one wave (64 / TAU blocks for
+// teams of fewer than 64 lanes), else one block.  Unit u's entries lie in
+// order from stage[u * unit_blocks * G] on, packed as (fp16 value << 16) |
+// place in the unit (at most 65536 elements), so that short blocks, which
+// hold an outlier or two each, share cache lines: staged block by block as
+// separate columns and values, a 14336 x 4096 weight in blocks of 128 with
+// 1.8 % outliers left two partly written lines per block, and reading them
+// back took half of the finish (45.5 us for that weight, now 16.5).
+__host__ __device__ constexpr int team_lanes(int64_t G) {  // TAU of launch_quantize, for G up to 2048
+  return G <= 16 ? 1 : G <= 64 ? 2 : G <= 128 ? 4 : G <= 256 ? 8 : G <= 512 ? 16 : G <= 1024 ? 32 : 64;
+}
+__host__ __device__ constexpr int unit_blocks(int64_t G) { return 64 / team_lanes(G); }
+
+// Row of block g (both below 2^31) in the tiled layout.
+__device__ __forceinline__ int64_t block_row(const QuantArgs& a, int64_t g) {
+  return a.bshift >= 0 ? g >> a.bshift : (int64_t)((uint32_t)g / (uint32_t)a.bpr);
+}
 
 // Up to kMaxQGroup weights of one block size quantized by one launch
 // (aq_quantize_grouped; aq_quantize is a group of one): workgroup b takes
@@ -217,29 +237,46 @@ __device__ float outlier_cut(f16 den, f16 thr) {
   return (float)bits_to_h((uint16_t)lo);
 }
 
-// Th for a team of TAU threads (the same value in every lane): lane j of the
-// team (j < 16) tests the bit pattern c0 - 8 + j, c0 = bits of fp16(thr * den).
+// Th for a team of TAU threads (the same value in every lane): its lanes test
+// consecutive bit patterns around c0 = bits of fp16(thr * den), 16 of them
+// (8 or 4 for teams of 8 or fewer lanes; lanes of teams of fewer than 4 test
+// several each), and the first that passes is the step.  For den positive
+// and finite, 0 / den = 0 and inf / den = inf settle the thresholds that all
+// or none pass.  Otherwise a passes once a / den > thr (1 + d), where d, half
+// a unit of thr, is between 2^-12 and 2^-11 relative, at most one unit of a:
+// the step lies between c0 and c0 + 2, so four patterns from c0 - 1 on hold
+// it.  (Four from c0 - 2 on missed it for one block in twenty, and with 16
+// blocks of 128 to a wave every second wave bisected: with the sums' exact
+// cases below, 1096 -> 787 VALU instructions a wave and 63 -> 51 us for a
+// 14336 x 4096 weight.)  Subnormal thresholds
+// and products may fall outside: those bisect.
 template <int TAU>
 __device__ float outlier_cut_team(f16 den, f16 thr) {
   const float fden = (float)den;
   if (!(fden > 0.0f) || isinf(fden)) return __builtin_nanf("");
-  if (outlier_literal(bits_to_h(0), den, thr)) return -1.0f;        // all are outliers
-  if (!outlier_literal(bits_to_h(0x7C00), den, thr)) return INFINITY;  // none
-  constexpr int W = TAU < 16 ? TAU : 16;
+  if (0.0f > (float)thr) return -1.0f;            // all are outliers
+  if (!(INFINITY > (float)thr)) return INFINITY;  // none
+  constexpr int W = TAU < 16 ? TAU : 16;   // lanes that test
+  constexpr int PL = W >= 4 ? 1 : 4 / W;   // patterns per lane
+  constexpr int below = W * PL == 4 ? 1 : W * PL / 2;
   constexpr int TL = TAU < 64 ? TAU : 64;  // team lanes within one wave
   const int lane = threadIdx.x & 63;
   const int ts = lane & ~(TL - 1);  // the team's first lane in this wave
   const int j = lane - ts;
   const float est = (float)thr * fden;
   const int c0 = est < 65504.0f ? (int)h_to_bits(rn_h(est)) : 0x7BFF;
-  const int cand = c0 - W / 2 + j;
-  // below 0 the test is false (checked at 0 above), past 0x7C00 true (checked at inf)
-  bool p = cand > 0x7C00 || (cand >= 0 && outlier_literal(bits_to_h((uint16_t)cand), den, thr));
-  p = p && j < W;
-  const uint64_t bal = __ballot(p);
-  const uint32_t bits = (uint32_t)(bal >> ts) & ((1u << W) - 1u);
+  uint32_t bits = 0;
+#pragma unroll
+  for (int k = 0; k < PL; k++) {
+    const int cand = c0 - below + k * W + j;
+    // below 0 the test is false (checked at 0 above), past 0x7C00 true (checked at inf)
+    bool p = cand > 0x7C00 || (cand >= 0 && outlier_literal(bits_to_h((uint16_t)cand), den, thr));
+    p = p && j < W;
+    const uint64_t bal = __ballot(p);
+    bits |= ((uint32_t)(bal >> ts) & ((1u << W) - 1u)) << (k * W);
+  }
   if (bits != 0 && !(bits & 1u)) {
-    const int first = c0 - W / 2 + __builtin_ctz(bits);  // smallest pattern that passes
+    const int first = c0 - below + __builtin_ctz(bits);  // smallest pattern that passes
     return (float)bits_to_h((uint16_t)(first - 1));
   }
   return outlier_cut(den, thr);
@@ -274,6 +311,22 @@ __device__ __forceinline__ void load_elems(Elems<E>& xs, const QuantArgs& a, int
       xs.p[e / 2] = pair;
     }
   }
+}
+
+// Where a team's outliers go in the stage: the unit's first element and the
+// team's first element in it.  *pre, the thread's place among its team's
+// outliers, becomes its place among the unit's.  Every lane of the wave
+// calls it (count 0 past the last block).
+struct UnitPlace {
+  int64_t base;
+  int at;
+};
+template <int TAU>
+__device__ __forceinline__ UnitPlace unit_place(int count, int64_t base, int64_t G, int* pre) {
+  if constexpr (TAU >= 64) return UnitPlace{base, 0};
+  *pre = wave_incl_scan_i32<64>(count) - count;
+  const int team = (int)(threadIdx.x & 63) / TAU;
+  return UnitPlace{base - team * G, team * (int)G};
 }
 
 // The rest of a block after its elements are loaded, for any block length:
@@ -330,7 +383,7 @@ __device__ __forceinline__ void finish_block_any(const QuantArgs& a, Elems<E>& x
   // where the thread's elements sit in the [rows, K] matrix (tiled layout)
   int64_t row = 0, col0 = 0;
   if (a.tiled) {
-    row = a.bpr == 1 ? g : g / a.bpr;
+    row = block_row(a, g);
     col0 = (g - row * a.bpr) * G + i0;
   }
 
@@ -389,9 +442,10 @@ __device__ __forceinline__ void finish_block_any(const QuantArgs& a, Elems<E>& x
   }
 
   // outlier compaction: team prefix sum, then the block's staging slot
-  const int cnt = __builtin_popcountll(omask);
+  const int cnt = gvalid ? __builtin_popcountll(omask) : 0;
   int total;
-  const int pre = team_excl_scan_i32<TAU>(cnt, lds_i, &total);
+  int pre = team_excl_scan_i32<TAU>(cnt, lds_i, &total);
+  const UnitPlace up = unit_place<TAU>(cnt, base, G, &pre);
   if (gvalid) {
     int k = pre;
     uint64_t m = omask;
@@ -401,8 +455,8 @@ __device__ __forceinline__ void finish_block_any(const QuantArgs& a, Elems<E>& x
       // the value from memory (an L2 hit): indexing the registers with a
       // run-time e would move them to scratch; padding elements are 0
       const int64_t j = base + i0 + e;
-      a.stage_col[base + k] = i0 + e;
-      a.stage_val[base + k] = j < a.numel ? a.x[j] : (uint16_t)0;
+      const uint32_t v = j < a.numel ? a.x[j] : (uint16_t)0;
+      a.stage[up.base + k] = (v << 16) | (uint32_t)(up.at + i0 + e);
       k++;
     }
     if (t == 0) {
@@ -446,9 +500,10 @@ __device__ __forceinline__ f16 std_of_var(double V, int64_t G) { return rn_h((fl
 //        roundings of u = 2^-24 per thread, so |S_f32 - S| <= d u sum|x|
 //        (the f64 sum across the team adds under 2^-46 relative), and
 //        sum|x| <= sqrt(G Q) by Cauchy-Schwarz;
-//   Q  = sum x^2 (products exact in f32, four f32 chains of E / 8 per
+//   Q  = sum x^2 (products exact in f32, four f32 chains of E / 4 per
 //        thread, then f32 across the team): a sum of non-negative terms
-//        with at most E / 8 + 2 + log2(TAU) roundings, within Q 2^-19.
+//        with at most n = E / 4 + 1 + log2(TAU) roundings of 2^-24 each
+//        (below 2^-19 in all), taken as n + 2 for what follows it.
 // mean16 is a monotone function of S, so when both ends of S_f32 +- errS
 // give the same mean16, that is the value the exact sum gives; std16 is a
 // monotone function of V = Q - S mu, accepted when both ends of V +- errV
@@ -469,6 +524,9 @@ __device__ __forceinline__ BlockStats block_stats_fast(Elems<E>& xs, int i0, con
   constexpr bool kSyncedTeams = TAU > 64 && NT / TAU > 1;
   constexpr int kDepth = E == 16 ? 4 : E == 32 ? 5 : 6;
   static_assert(E == 16 || E == 32 || E == 64, "tree depth");
+  constexpr int kQRound = E / 4 + 1 + (TAU <= 1 ? 0 : TAU <= 2 ? 1 : TAU <= 4 ? 2 : TAU <= 8 ? 3 : TAU <= 16 ? 4
+                                       : TAU <= 32 ? 5 : TAU <= 64 ? 6 : TAU <= 128 ? 7 : TAU <= 256 ? 8
+                                       : TAU <= 512 ? 9 : 10);
   const int64_t G = a.G;
   // padding elements are zeros: every E elements enter the sums
   float sp[E / 2];
@@ -486,6 +544,7 @@ __device__ __forceinline__ BlockStats block_stats_fast(Elems<E>& xs, int i0, con
   }
   double Sf = (double)sp[0];
   float Qf = (q[0] + q[1]) + (q[2] + q[3]);
+  const float q_thread = Qf;
   // the block's first use of lds_d / lds_f (one block per team and workgroup)
   team_sum_f64_f32<TAU, true>(Sf, Qf, lds_d, lds_f);
   const double Q = (double)Qf;
@@ -493,7 +552,17 @@ __device__ __forceinline__ BlockStats block_stats_fast(Elems<E>& xs, int i0, con
   // products' roundings, (1 + 2^-20) the square root's one ulp and the last
   // rounding (G Q stays below 2^47: no overflow; an inf or NaN propagates)
   const float absum = __builtin_amdgcn_sqrtf((float)G * Qf * (1.0f + 0x1p-14f)) * (1.0f + 0x1p-20f);
-  const double errS = (double)(kDepth + 1) * 0x1p-24 * (double)absum + fabs(Sf) * 0x1p-50;
+  double errS = (double)(kDepth + 1) * 0x1p-24 * (double)absum + fabs(Sf) * 0x1p-50;
+  // Every fp16 is a multiple of 2^-24, so partial sums of magnitude up to 1
+  // are exact in f32, and a thread's are when its sum|x| <= sqrt(E q) <= 1
+  // (q here a thread's own sum of squares, off by 2^-19 at most).  Weights of
+  // a model's size pass unless a thread holds a large outlier: with 16 teams
+  // of 128 elements to a wave, one of them met an open bracket in every
+  // fifth wave otherwise.
+  if constexpr (TAU <= 16) {
+    const uint64_t bal = __ballot(!((float)E * q_thread <= 0.999f));
+    if (((bal >> (threadIdx.x & 63 & ~(TAU - 1))) & ((1ull << TAU) - 1)) == 0) errS = 0.0;
+  }
   // the bracket's ends as (Sf -+ errS2) * RN64(1 / G): three f64 roundings
   // move a product by at most 3.1 * 2^-53 of |Sf| + errS2, which the extra
   // |Sf| 2^-49 and errS 2^-48 exceed, so lo_t <= (Sf - errS) / G and
@@ -516,10 +585,10 @@ __device__ __forceinline__ BlockStats block_stats_fast(Elems<E>& xs, int i0, con
   bool open = true;
   if (G >= 2) {
     // |S * mu| <= Q (Cauchy-Schwarz): every rounding below, and mu taken as
-    // S * RN64(1 / G), stays far inside the Q 2^-16 term
+    // S * RN64(1 / G), stays far inside one of the two spare units of Q's term
     const double mu = S * a.inv_g;
     const double V = Q - S * mu;
-    const double err = Q * 0x1p-16 + (2.0 * fabs(S) + dS) * dS * a.inv_g + fabs(V) * 0x1p-50;
+    const double err = Q * ((kQRound + 2) * 0x1p-24) + (2.0 * fabs(S) + dS) * dS * a.inv_g + fabs(V) * 0x1p-50;
     // sqrt((V -+ err) / (G - 1)) in f32 with c = RN32(1 / (G - 1)): the
     // conversions, the product and the square root (one ulp) stay within
     // 2^-22 relative, so the 2^-20 pulls put ylo below and yhi above the
@@ -705,7 +774,9 @@ __device__ __forceinline__ void finish_block_fast(const QuantArgs& a, Elems<E>& 
   // the block's first use of lds_i, its counts in the first NWT words, the
   // absmax in the next NWT
   constexpr int NWT = TAU > 64 ? TAU / 64 : 1;
-  const int pre = team_scan_max<TAU, true>(nout, &amax, lds_i, reinterpret_cast<float*>(lds_i + NWT), &total);
+  if (!gvalid) nout = 0;
+  int pre = team_scan_max<TAU, true>(nout, &amax, lds_i, reinterpret_cast<float*>(lds_i + NWT), &total);
+  const UnitPlace up = unit_place<TAU>(nout, base, G, &pre);
   if (gvalid) {
     int k = pre;
 #pragma unroll
@@ -727,8 +798,8 @@ __device__ __forceinline__ void finish_block_fast(const QuantArgs& a, Elems<E>& 
         // hit): indexing the registers with a run-time e would move them to
         // scratch
         const int64_t jj = base + i0 + e;
-        a.stage_col[base + k] = i0 + e;
-        a.stage_val[base + k] = staged ? staged[staged_index<E>(unit_e0 + e)] : (jj < a.numel ? a.x[jj] : (uint16_t)0);
+        const uint32_t v = staged ? staged[staged_index<E>(unit_e0 + e)] : (jj < a.numel ? a.x[jj] : (uint16_t)0);
+        a.stage[up.base + k] = (v << 16) | (uint32_t)(up.at + i0 + e);
         k++;
       }
     }
@@ -749,7 +820,7 @@ __device__ __forceinline__ void finish_block_fast(const QuantArgs& a, Elems<E>& 
 
   int64_t row = 0, col0 = 0;  // where the thread's elements sit in the [rows, K] matrix (tiled layout)
   if (a.tiled) {
-    row = a.bpr == 1 ? g : g / a.bpr;
+    row = block_row(a, g);
     col0 = (g - row * a.bpr) * G + i0;
   }
   // Where the thread's first 16 codes go; group v of 16 follows at v * 256
@@ -1025,85 +1096,91 @@ __global__ __launch_bounds__(1024) void scan_small_kernel(ScanGroup sg) {
 
 // ---- gather the staged outliers into the ascending list
 
-template <int TPB>
-__global__ __launch_bounds__(256) void gather_kernel(const int32_t* off, int64_t nblocks, int64_t G, int64_t K,
-                                                     const int32_t* stage_col, const uint16_t* stage_val,
-                                                     int64_t* flat_idx, uint16_t* vals, int32_t* cols) {
+// TPU lanes per staging unit of ub blocks.
+template <int TPU>
+__global__ __launch_bounds__(256) void gather_kernel(const int32_t* off, int64_t nblocks, int64_t G, int ub,
+                                                     uint32_t K, const uint32_t* stage, int64_t* flat_idx,
+                                                     uint16_t* vals, int32_t* cols) {
   const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t g = gid / TPB;
-  const int lane = (int)(gid % TPB);
-  if (g >= nblocks) return;
-  const int32_t o = off[g];
-  const int32_t n = off[g + 1] - o;
-  const int64_t base = g * G;
-  for (int j = lane; j < n; j += TPB) {
-    const int64_t flat = base + stage_col[base + j];
+  const int64_t b0 = gid / TPU * ub;
+  const int lane = (int)(gid % TPU);
+  if (b0 >= nblocks) return;
+  const int32_t o = off[b0];
+  const int32_t n = off[min(b0 + ub, nblocks)] - o;
+  const int64_t base = b0 * G;
+  for (int j = lane; j < n; j += TPU) {
+    const uint32_t e = stage[base + j];
+    const uint32_t flat = (uint32_t)base + (e & 0xFFFFu);  // below 2^31 (quantize_args)
     flat_idx[o + j] = flat;
-    vals[o + j] = stage_val[base + j];
+    vals[o + j] = (uint16_t)(e >> 16);
     if (cols) cols[o + j] = (int32_t)(flat % K);
   }
 }
 
 // ---- the flat list and the 16 x 64 block lists in one pass
 
-// Entries of one tile row straight from the quantize workspace: block g's
-// outliers are staged at stage_col / stage_val[g G .. g G + n_g - 1]
-// (columns within the block, ascending), and its first entry's index is
-// off[g].  In the counting pass each entry also goes to the flat list, as
+// Entries of one tile row straight from the quantize workspace (staged by
+// unit, see unit_blocks; a unit may begin before the tile row or end behind
+// it).  In the counting pass each entry also goes to the flat list, as
 // gather_kernel writes it.
 struct WsTileSrc {
   int rs[17];            // the tile row's row starts, off[(16 rb + r) bpr]
   const int32_t* off;    // block offsets
-  const int* loff;       // the tile row's 16 bpr + 1 block offsets in LDS, or null (read off)
-  int64_t g0;            // the tile row's first block
-  int bpr;               // blocks per row, K / G
-  int64_t G;
-  const int32_t* stage_col;
-  const uint16_t* stage_val;
+  const int* loff;       // the tile row's nu + 1 unit starts in LDS, or null (read off)
+  int64_t u0;            // the tile row's first unit
+  int64_t nblocks;
+  int nu;                // its units
+  int ub;                // blocks per unit
+  int rows;              // each of the 16 rows is a unit
+  int64_t unit_len;      // elements per unit, ub G
+  int64_t row0;          // the tile row's first element
+  uint32_t K;
+  const uint32_t* stage;
   int64_t* flat_idx;
   uint16_t* vals;
   int32_t* cols;
-  __device__ __forceinline__ int block_start(int b) const { return loff ? loff[b] : off[g0 + b]; }
+  __device__ __forceinline__ int unit_start(int u) const {
+    return loff ? loff[u] : off[min((u0 + u) * ub, nblocks)];
+  }
   __device__ __forceinline__ aq::TileEnt operator()(int i, bool first) const {
-    int b, r, o;
-    if (bpr == 1) {
+    int u, o;
+    if (rows) {
       // the row and its start by a select chain (an index into rs would move
       // the array to scratch memory)
-      r = 0;
+      u = 0;
       o = rs[0];
 #pragma unroll
       for (int k = 1; k < 16; k++)
         if (i >= rs[k]) {
-          r = k;
+          u = k;
           o = rs[k];
         }
-      b = r;
     } else {
-      // the last block of the tile row starting at or before entry i (blocks
-      // may be empty): block_start(0) <= i < block_start(16 bpr)
-      int lo = 1, hi = 16 * bpr;
+      // the last unit starting at or before entry i (units may be empty):
+      // unit_start(0) <= i < unit_start(nu)
+      int lo = 1, hi = nu;
       while (lo < hi) {
         const int mid = (lo + hi) >> 1;
-        if (block_start(mid) <= i)
+        if (unit_start(mid) <= i)
           lo = mid + 1;
         else
           hi = mid;
       }
-      b = lo - 1;
-      r = b / bpr;
-      o = block_start(b);
+      u = lo - 1;
+      o = unit_start(u);
     }
-    const int64_t g = g0 + b;
-    const int64_t at = g * G + (i - o);
-    const int sc = stage_col[at];
-    const uint32_t v = stage_val[at];
-    const int col = (b - r * bpr) * (int)G + sc;
+    const int64_t base = (u0 + u) * unit_len;
+    const uint32_t e = stage[base + (i - o)];
+    const int64_t flat = base + (e & 0xFFFFu);
+    const uint32_t rel = (uint32_t)(flat - row0);  // below 16 K
+    const int r = rows ? u : (int)(rel / K);
+    const int col = (int)(rel - (uint32_t)r * K);
     if (first) {
-      flat_idx[i] = g * G + sc;
-      vals[i] = (uint16_t)v;
+      flat_idx[i] = flat;
+      vals[i] = (uint16_t)(e >> 16);
       cols[i] = col;
     }
-    return aq::TileEnt{r, col, v};
+    return aq::TileEnt{r, col, e >> 16};
   }
 };
 
@@ -1113,8 +1190,7 @@ struct WsTileSrc {
 // lists' end and their 64 padding entries.
 struct FinishMember {
   const int32_t* off;
-  const int32_t* stage_col;
-  const uint16_t* stage_val;
+  const uint32_t* stage;
   int64_t* flat_idx;
   uint16_t* vals;
   int32_t* cols;
@@ -1127,15 +1203,24 @@ struct FinishGroup {
   FinishMember m[kMaxQGroup];
   int first[kMaxQGroup + 1];
   int count;
-  int bpr, nch, loff_lds;
+  int bpr, nch, loff_lds, ub;
+  int raise;  // the tile rows raise tile_max themselves
   int64_t G;
 };
 
-// LDS: 33 * nch ints, and with loff_lds the tile row's block offsets after
-// them.  NT threads per tile row: 128 for rows up to 128 chunks (a tile row of
-// such weights holds a few hundred entries, and the small workgroups let a
-// layer's tile rows all be resident at once), 256 for wider ones.
-template <int NT>
+// Units that overlap a tile row of 16 bpr blocks: at most one more than fit
+// when the tile rows do not start on unit boundaries.
+__host__ __device__ constexpr int tile_row_units(int bpr, int ub) {
+  return 16 * bpr % ub == 0 ? 16 * bpr / ub : 16 * bpr / ub + 2;
+}
+
+// LDS: 33 * nch ints, and with loff_lds the tile row's unit starts after
+// them.  NT threads per tile row, each keeping its first REGS entries in
+// registers between the two passes of the sort: 128 x 4 where a tile row
+// holds a few hundred entries (the small workgroups let a layer's tile rows
+// all be resident at once), 256 x 8 for crowded ones, whose entries would
+// otherwise be searched for and read twice.
+template <int NT, int REGS>
 __global__ __launch_bounds__(NT) void finish_tiles_kernel(FinishGroup fg) {
   extern __shared__ int sm[];
   __shared__ int part[NT / 64];
@@ -1155,23 +1240,29 @@ __global__ __launch_bounds__(NT) void finish_tiles_kernel(FinishGroup fg) {
   WsTileSrc src;
 #pragma unroll
   for (int r = 0; r <= 16; r++) src.rs[r] = m.off[(int64_t)(rb * 16 + r) * bpr];
+  const int64_t g0 = (int64_t)rb * 16 * bpr;  // the tile row's first block
   src.off = m.off;
   src.loff = nullptr;
-  src.g0 = (int64_t)rb * 16 * bpr;
-  src.bpr = bpr;
-  src.G = fg.G;
-  src.stage_col = m.stage_col;
-  src.stage_val = m.stage_val;
+  src.ub = fg.ub;
+  src.u0 = g0 / fg.ub;
+  src.nu = (int)((g0 + 16 * bpr + fg.ub - 1) / fg.ub - src.u0);
+  src.nblocks = (int64_t)m.nrb * 16 * bpr;
+  src.rows = bpr == 1 && fg.ub == 1;
+  src.unit_len = fg.ub * fg.G;
+  src.row0 = g0 * fg.G;
+  src.K = (uint32_t)nch * 64;
+  src.stage = m.stage;
   src.flat_idx = m.flat_idx;
   src.vals = m.vals;
   src.cols = m.cols;
   if (fg.loff_lds) {
     int* l = sm + 33 * nch;
-    for (int k = t; k <= 16 * bpr; k += NT) l[k] = m.off[src.g0 + k];
+    for (int k = t; k <= src.nu; k += NT) l[k] = src.unit_start(k);
     __syncthreads();
     src.loff = l;
   }
-  aq::tile_row_sort<NT>(src, rb, nch, src.rs[0], src.rs[16], sm, part, m.tile_ptr, m.tile_ent, m.tile_max);
+  aq::tile_row_sort<NT, REGS>(src, rb, nch, src.rs[0], src.rs[16], sm, part, m.tile_ptr, m.tile_ent,
+                              fg.raise ? m.tile_max : nullptr);
 }
 
 // ---- calculate_zscore_manual of one block of n elements
@@ -1210,6 +1301,7 @@ template <int TAU, int E>
 hipError_t launch_quantize_t(QuantGroup q, hipStream_t stream) {
   constexpr int NT = TAU > kWG ? TAU : kWG;
   constexpr int TEAMS = NT / TAU;
+  if (unit_blocks(q.m[0].G) != (TAU < 64 ? 64 / TAU : 1)) return hipErrorInvalidValue;  // the staging layout
   q.first[0] = 0;
   for (int i = 0; i < q.count; i++) q.first[i + 1] = q.first[i] + aq::ceil_div(q.m[i].nblocks, TEAMS);
   for (int i = q.count + 1; i <= kMaxQGroup; i++) q.first[i] = q.first[q.count];
@@ -1270,25 +1362,18 @@ hipError_t launch_zscore_t(const uint16_t* x, int64_t n, float eps, uint16_t* z,
 }
 
 struct Workspace {
-  int32_t* stage_col;
-  uint16_t* stage_val;
+  uint32_t* stage;
   int32_t* partial;
 };
 
 int64_t align256(int64_t b) { return (b + 255) / 256 * 256; }
 
-Workspace carve(void* ws, int64_t padded, int64_t nblocks) {
-  char* p = (char*)ws;
-  Workspace w;
-  w.stage_col = (int32_t*)p;
-  p += align256(padded * 4);
-  w.stage_val = (uint16_t*)p;
-  p += align256(padded * 2);
-  w.partial = (int32_t*)p;
-  (void)nblocks;
-  return w;
+Workspace carve(void* ws, int64_t padded) {
+  return Workspace{(uint32_t*)ws, (int32_t*)((char*)ws + align256(padded * 4))};
 }
 
+// (2 bytes an element more than the stage takes: the size has been this much
+// for callers that compute with it)
 int64_t workspace_bytes(int64_t padded, int64_t nblocks) {
   return align256(padded * 4) + align256(padded * 2) + align256((aq::ceil_div(nblocks, kScanChunk) + 1) * 4);
 }
@@ -1326,7 +1411,7 @@ static int quantize_args(const void* x, int64_t numel, int64_t G, uint16_t z_thr
   if (ws_bytes < workspace_bytes(padded, nblocks))
     return aq::set_error(AQ_EWORKSPACE, "aq_quantize: workspace of %lld bytes, %lld needed", (long long)ws_bytes,
                          (long long)workspace_bytes(padded, nblocks));
-  const Workspace w = carve(workspace, padded, nblocks);
+  const Workspace w = carve(workspace, padded);
   QuantArgs a;
   a.x = (const uint16_t*)x;
   a.numel = numel;
@@ -1339,13 +1424,13 @@ static int quantize_args(const void* x, int64_t numel, int64_t G, uint16_t z_thr
   a.K = K;
   a.nchunks = K / 128;
   a.bpr = a.tiled ? K / G : 1;
+  a.bshift = (a.bpr & (a.bpr - 1)) ? -1 : __builtin_ctzll((uint64_t)a.bpr);
   a.inv_g = 1.0 / (double)G;
   a.inv_g1 = G >= 2 ? (float)(1.0 / (double)(G - 1)) : 0.0f;
   a.codes = (uint8_t*)codes;
   a.scales = (uint16_t*)scales;
   a.block_cnt = block_off;
-  a.stage_col = w.stage_col;
-  a.stage_val = w.stage_val;
+  a.stage = w.stage;
   *out = a;
   *wout = w;
   return AQ_OK;
@@ -1430,16 +1515,18 @@ extern "C" int aq_quantize_finish(int64_t numel, int64_t G, int64_t K, const int
     return aq::set_error(AQ_EWORKSPACE, "aq_quantize_finish: workspace too small");
   if (nnz == 0) return AQ_OK;
   AQ_CHECK_ARG(flat_idx && vals && block_off, "aq_quantize_finish: null pointer argument");
-  Workspace w = carve((void*)workspace, padded, nblocks);
+  Workspace w = carve((void*)workspace, padded);
   hipStream_t s = (hipStream_t)stream;
-  if (G >= 256) {
-    const int64_t grid = aq::ceil_div(nblocks * 64, 256);
-    hipLaunchKernelGGL((gather_kernel<64>), dim3((unsigned)grid), dim3(256), 0, s, block_off, nblocks, G, K,
-                       w.stage_col, w.stage_val, flat_idx, (uint16_t*)vals, cols);
+  const int ub = unit_blocks(G);
+  const int64_t nunits = aq::ceil_div(nblocks, ub);
+  // an outlier index is below 2^31, so any larger K leaves it as it is
+  const uint32_t k32 = (uint32_t)std::min<int64_t>(K, (int64_t)1 << 31);
+  if (ub * G >= 1024) {
+    hipLaunchKernelGGL((gather_kernel<16>), dim3((unsigned)aq::ceil_div(nunits * 16, 256)), dim3(256), 0, s, block_off,
+                       nblocks, G, ub, k32, w.stage, flat_idx, (uint16_t*)vals, cols);
   } else {
-    const int64_t grid = aq::ceil_div(nblocks, 256);
-    hipLaunchKernelGGL((gather_kernel<1>), dim3((unsigned)grid), dim3(256), 0, s, block_off, nblocks, G, K,
-                       w.stage_col, w.stage_val, flat_idx, (uint16_t*)vals, cols);
+    hipLaunchKernelGGL((gather_kernel<4>), dim3((unsigned)aq::ceil_div(nunits * 4, 256)), dim3(256), 0, s, block_off,
+                       nblocks, G, ub, k32, w.stage, flat_idx, (uint16_t*)vals, cols);
   }
   AQ_LAUNCH_CHECK("aq_quantize_finish: gather launch");
   return AQ_OK;
@@ -1461,11 +1548,10 @@ static int finish_tiles_member(const char* fn, int64_t numel, int64_t G, int64_t
     return aq::set_error(AQ_EWORKSPACE, "%s: workspace too small", fn);
   AQ_CHECK_ARG(block_off && workspace && tile_ptr && tile_ent && (nnz == 0 || (flat_idx && vals && cols)),
                "%s: null pointer argument", fn);
-  const Workspace w = carve((void*)workspace, numel, nblocks);
+  const Workspace w = carve((void*)workspace, numel);
   FinishMember m;
   m.off = block_off;
-  m.stage_col = w.stage_col;
-  m.stage_val = w.stage_val;
+  m.stage = w.stage;
   m.flat_idx = flat_idx;
   m.vals = (uint16_t*)vals;
   m.cols = cols;
@@ -1477,24 +1563,42 @@ static int finish_tiles_member(const char* fn, int64_t numel, int64_t G, int64_t
   return AQ_OK;
 }
 
-// One launch for the group's members (all of one block size G and row length K).
-static int launch_finish_tiles(FinishGroup& fg, int64_t G, int64_t K, const char* fn, hipStream_t s) {
+// One launch for the group's members (all of one block size G and row
+// length K); most: the largest outlier count of a member per tile row.
+static int launch_finish_tiles(FinishGroup& fg, int64_t G, int64_t K, int64_t most, const char* fn, hipStream_t s) {
   const int64_t nch = K / 64, bpr = K / G;
   fg.G = G;
   fg.bpr = (int)bpr;
   fg.nch = (int)nch;
+  fg.ub = unit_blocks(G);
   fg.first[0] = 0;
   for (int i = 0; i < fg.count; i++) fg.first[i + 1] = fg.first[i] + fg.m[i].nrb + 1;
   for (int i = fg.count + 1; i <= kMaxQGroup; i++) fg.first[i] = fg.first[fg.count];
-  // the tile row's block offsets go to LDS when the sort leaves room (64 KiB in all)
-  const int64_t sort_ints = 33 * nch;
-  fg.loff_lds = bpr > 1 && sort_ints + 16 * bpr + 1 <= 16384;
-  const size_t lds = (size_t)(sort_ints + (fg.loff_lds ? 16 * bpr + 1 : 0)) * sizeof(int);
-  if (nch <= 128)
-    hipLaunchKernelGGL(finish_tiles_kernel<128>, dim3((unsigned)fg.first[fg.count]), dim3(128), lds, s, fg);
+  // the tile row's unit starts go to LDS when the sort leaves room (64 KiB in all)
+  const int64_t sort_ints = 33 * nch, units = tile_row_units((int)bpr, fg.ub);
+  fg.loff_lds = !(bpr == 1 && fg.ub == 1) && sort_ints + units + 1 <= 16384;
+  const size_t lds = (size_t)(sort_ints + (fg.loff_lds ? units + 1 : 0)) * sizeof(int);
+  const dim3 grid((unsigned)fg.first[fg.count]);
+  fg.raise = fg.first[fg.count] <= aq::kRaiseTileRows;
+  if (most > 768)
+    hipLaunchKernelGGL((finish_tiles_kernel<256, 8>), grid, dim3(256), lds, s, fg);
+  else if (nch <= 128 && most <= 448)
+    hipLaunchKernelGGL((finish_tiles_kernel<128, 4>), grid, dim3(128), lds, s, fg);
   else
-    hipLaunchKernelGGL(finish_tiles_kernel<256>, dim3((unsigned)fg.first[fg.count]), dim3(256), lds, s, fg);
+    hipLaunchKernelGGL((finish_tiles_kernel<256, 4>), grid, dim3(256), lds, s, fg);
   AQ_LAUNCH_CHECK(fn);
+  aq::TileMaxGroup tm{};
+  static_assert(kMaxQGroup <= aq::kMaxTileMax, "one launch for the group");
+  bool any = false;
+  for (int i = 0; i < fg.count; i++) {
+    tm.tile_ptr[i] = fg.m[i].tile_ptr;
+    tm.n[i] = (int64_t)fg.m[i].nrb * nch;
+    tm.tile_max[i] = fg.m[i].tile_max;
+    any = any || fg.m[i].tile_max;
+  }
+  if (!any || fg.raise) return AQ_OK;
+  const hipError_t e = aq::launch_tile_max(tm, fg.count, s);
+  if (e != hipSuccess) return aq::check_hip(e, fn);
   return AQ_OK;
 }
 
@@ -1527,7 +1631,7 @@ extern "C" int aq_quantize_finish_tiles(int64_t numel, int64_t G, int64_t K, con
     return finish_tiles_wide(numel, G, K, block_off, nnz, workspace, ws_bytes, flat_idx, vals, cols, tile_ptr,
                              tile_ent, tile_max, fn, s);
   fg.count = 1;
-  return launch_finish_tiles(fg, G, K, fn, s);
+  return launch_finish_tiles(fg, G, K, nnz / fg.m[0].nrb, fn, s);
 }
 
 extern "C" int aq_quantize_finish_tiles_grouped(int64_t count, const int64_t* numels, int64_t G, int64_t K,
@@ -1542,11 +1646,13 @@ extern "C" int aq_quantize_finish_tiles_grouped(int64_t count, const int64_t* nu
                    tile_ents,
                "%s: null pointer argument", fn);
   FinishGroup fg{};
+  int64_t most = 0;
   for (int i = 0; i < (int)count; i++) {
     const int rc = finish_tiles_member(fn, numels[i], G, K, block_offs[i], nnzs[i], workspaces[i], ws_bytes[i],
                                        flat_idx[i], vals[i], cols[i], tile_ptrs[i], tile_ents[i],
                                        tile_max ? tile_max + i : nullptr, &fg.m[i]);
     if (rc != AQ_OK) return rc;
+    most = std::max(most, nnzs[i] / fg.m[i].nrb);
   }
   hipStream_t s = (hipStream_t)stream;
   if (K / 64 > aq::kTileRowsMaxChunks) {
@@ -1559,7 +1665,7 @@ extern "C" int aq_quantize_finish_tiles_grouped(int64_t count, const int64_t* nu
     return AQ_OK;
   }
   fg.count = (int)count;
-  return launch_finish_tiles(fg, G, K, fn, s);
+  return launch_finish_tiles(fg, G, K, most, fn, s);
 }
 
 extern "C" int aq_zscore(const void* x, int64_t n, float eps, void* z, void* stats, void* stream) {

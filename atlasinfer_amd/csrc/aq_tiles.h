@@ -12,7 +12,7 @@
 // starts; an entry's place is its block's start, the entries of its chunk in
 // the rows above, and its rank in its (row, chunk) run, which is contiguous
 // in the row's sorted columns: its index minus the run's first.  A thread's
-// first kTileRowsRegs entries stay in registers between the two passes.
+// first REGS entries stay in registers between the two passes.
 #pragma once
 
 #include "aq_common.h"
@@ -20,7 +20,6 @@
 namespace aq {
 
 constexpr int kTileRowsMaxChunks = 480;  // K <= 30720: 33 * 480 ints of LDS (63360 bytes)
-constexpr int kTileRowsRegs = 4;
 
 // Position of row r (0..15), column k (0..63) in a block's entry: r << 6 | k.
 __device__ __forceinline__ uint32_t block_position(int r, int k) { return ((uint32_t)r << 6) | (uint32_t)k; }
@@ -39,8 +38,7 @@ __device__ __forceinline__ int lower_bound_i32(const int32_t* a, int lo, int hi,
 // Raise *p to at least v.  Many workgroups raise one word: a relaxed read
 // first skips the atomic when the word is already that large (it only
 // grows, so skipping keeps the maximum), since atomics on one address are
-// serialized at the L2 (one per wave over a layer's tile rows took three
-// quarters of the tile-row sort's launch).
+// serialized in memory at about 8 ns each.
 __device__ __forceinline__ void raise_to(int32_t* p, int v) {
   if (v > __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(p, v);
 }
@@ -77,7 +75,7 @@ struct CsrTileSrc {
 // tile_ptr[rb * nch + c] for every chunk and the entries, and raises
 // *tile_max (if not null) to the largest block.  Every thread of the
 // workgroup calls it.
-template <int NT, typename Src>
+template <int NT, int REGS, typename Src>
 __device__ __forceinline__ void tile_row_sort(const Src& src, int rb, int nch, int p0, int p1, int* sm, int* part,
                                               int32_t* tile_ptr, uint32_t* tile_ent, int32_t* tile_max) {
   static_assert(NT == 128 || NT == 256, "workgroup size");
@@ -86,9 +84,9 @@ __device__ __forceinline__ void tile_row_sort(const Src& src, int rb, int nch, i
   int* bstart = sm + 32 * nch;  // [nch]: block totals, then block starts
   const int t = threadIdx.x;
   // this thread's first entries: their loads go out before the LDS is cleared
-  TileEnt ce[kTileRowsRegs];
+  TileEnt ce[REGS];
 #pragma unroll
-  for (int k = 0; k < kTileRowsRegs; k++) {
+  for (int k = 0; k < REGS; k++) {
     const int i = p0 + t + NT * k;
     ce[k] = i < p1 ? src(i, true) : TileEnt{0, 0, 0u};
   }
@@ -98,7 +96,7 @@ __device__ __forceinline__ void tile_row_sort(const Src& src, int rb, int nch, i
   }
   __syncthreads();
 #pragma unroll
-  for (int k = 0; k < kTileRowsRegs; k++) {
+  for (int k = 0; k < REGS; k++) {
     const int i = p0 + t + NT * k;
     if (i < p1) {
       const int b = ce[k].r * nch + (ce[k].col >> 6);
@@ -106,7 +104,7 @@ __device__ __forceinline__ void tile_row_sort(const Src& src, int rb, int nch, i
       atomicMin(&first[b], i);
     }
   }
-  for (int i = p0 + t + NT * kTileRowsRegs; i < p1; i += NT) {
+  for (int i = p0 + t + NT * REGS; i < p1; i += NT) {
     const TileEnt e = src(i, true);
     const int b = e.r * nch + (e.col >> 6);
     atomicAdd(&cnt[b], 1);
@@ -154,22 +152,22 @@ __device__ __forceinline__ void tile_row_sort(const Src& src, int rb, int nch, i
   }
   __syncthreads();
 #pragma unroll
-  for (int k = 0; k < kTileRowsRegs; k++) {
+  for (int k = 0; k < REGS; k++) {
     const int i = p0 + t + NT * k;
     if (i < p1) {
       const int c = ce[k].col >> 6, b = ce[k].r * nch + c;
       tile_ent[p0 + bstart[c] + cnt[b] + (i - first[b])] = (ce[k].val << 16) | block_position(ce[k].r, ce[k].col - c * 64);
     }
   }
-  for (int i = p0 + t + NT * kTileRowsRegs; i < p1; i += NT) {
+  for (int i = p0 + t + NT * REGS; i < p1; i += NT) {
     const TileEnt e = src(i, false);
     const int c = e.col >> 6, b = e.r * nch + c;
     tile_ent[p0 + bstart[c] + cnt[b] + (i - first[b])] = (e.val << 16) | block_position(e.r, e.col - c * 64);
   }
-  // the largest block of the tile row: wave maxima through LDS (part is
-  // free again after the barrier), one raise per workgroup
-  for (int d = 32; d >= 1; d >>= 1) mx = max(mx, __shfl_xor(mx, d));
   if (tile_max) {
+    // wave maxima through LDS (part is free again after the barrier), one
+    // raise per workgroup
+    for (int d = 32; d >= 1; d >>= 1) mx = max(mx, __shfl_xor(mx, d));
     __syncthreads();
     if ((t & 63) == 0) part[t >> 6] = mx;
     __syncthreads();
@@ -180,6 +178,23 @@ __device__ __forceinline__ void tile_row_sort(const Src& src, int rb, int nch, i
     }
   }
 }
+
+// The largest block counts of up to kMaxTileMax block lists, raised into
+// each list's word from its finished tile_ptr (n blocks): a launch of its
+// own, a few workgroups a list, for launches of more than kRaiseTileRows tile
+// rows.  Raised by the sort's workgroups, which are all resident at once and
+// so all find the old value, the atomics on one word (8 ns each, in memory)
+// took longer than the sort: a layer's six weights, 2432 tile rows, 31.5 us
+// with them, 10.5 without, and this launch takes 3.8.  Fewer tile rows raise
+// it themselves, which costs less than a launch.  Defined in aq_layout.hip.
+constexpr int kRaiseTileRows = 320;
+constexpr int kMaxTileMax = 8;
+struct TileMaxGroup {
+  const int32_t* tile_ptr[kMaxTileMax];
+  int64_t n[kMaxTileMax];
+  int32_t* tile_max[kMaxTileMax];  // null: skipped
+};
+hipError_t launch_tile_max(const TileMaxGroup& g, int count, hipStream_t stream);
 
 // The block lists from CSR lists whose row r starts at row_ptr[r * rstride]
 // (rstride 1: a CSR row pointer; K / G: the block offsets of a weight whose
