@@ -39,7 +39,7 @@ FLAGS = [
 # per-file additions: the quantized-linear kernels keep MFMA accumulators in
 # ordinary VGPRs (the accumulator-register form made the compiler shuffle
 # accumulators between register files inside the K loop)
-FILE_FLAGS = {"aq_qlinear.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+FILE_FLAGS = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form=1"] for f in ("aq_qlinear.hip", "aq_qlinear_mid.hip")}
 
 
 def _compile(src: str) -> str:

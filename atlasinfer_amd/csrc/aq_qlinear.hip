@@ -75,6 +75,7 @@ constexpr int kGemvMaxM = 64;   // larger M takes the GEMM
 // faster on the GEMV)
 constexpr int kGemvShortMaxM = 32;
 constexpr int kGemvShortRows = 384;
+constexpr int kGemvTallRows = 768;
 constexpr int kGemvXMinM = 6;   // from here on the GEMV shares x through LDS (qlinear_gemv_x_kernel)
 constexpr int kGemvUnroll = 2;  // 128-wide K chunks per wave with loads in flight together
 constexpr int kGemvDirectMaxM = kGemvXMinM - 1;  // rows of x qlinear_gemv_kernel takes
@@ -1976,7 +1977,12 @@ extern "C" int64_t aq_qlinear_workspace_size(int64_t M, int64_t N, int64_t K) {
   return tail_bytes;
 }
 
-
+extern "C" int64_t aq_qlinear_decode_workspace_size(int64_t M, int64_t N, int64_t K) {
+  if (N <= 0 || K < 128 || K % 128 || M < kMidMinM || M > kMidMaxM) return 0;
+  if (N / 16 >= kGemvShortRows && N / 16 < kGemvTallRows) return 0;
+  const int split = mid_split(&N, 1, K);
+  return split > 1 ? split * M * N * 4 : 0;
+}
 
 // aq_qlinear_decode's additions to a grouped launch
 struct DecodeFuse {
@@ -2088,6 +2094,35 @@ static int qlinear_grouped_impl(const void* x, int64_t M, int64_t K, int fmt, in
   bool have_lists = tile_ptrs && tile_ents && tile_maxes;
   for (int i = 0; i < count && have_lists; i++) have_lists = tile_ptrs[i] && tile_ents[i];
   const bool gemv = M <= kGemvShortMaxM || (M <= kGemvMaxM && (blocks >= kGemvShortRows || !have_lists));
+  // Decode steps of 33 rows of x or more, given the block lists: short grids
+  // (below 384 tile rows) and tall ones (768 or more) split K over workgroups (aq_qlinear_mid.hip): at M = 64
+  // o_proj 25 -> 18.4 us and down_proj 90 -> 31 in a decode step, gate+up
+  // 54.5 -> 47.  Between them the shared-x GEMV stays ahead (q/k/v 22.3
+  // against 24.5, [8192, 2048] 14.6 against 19).
+  if (fz && M >= kMidMinM && M <= kMidMaxM && (blocks < kGemvShortRows || blocks >= kGemvTallRows) &&
+      tile_ptrs && tile_ents) {
+    const bool pair = a.mat[0].act == 2;
+    bool lists = true;
+    int64_t outs = 0;
+    for (int i = 0; i < count; i++) {
+      lists = lists && tile_ptrs[i] && tile_ents[i];
+      outs += M * Ns[i];
+    }
+    int split = mid_split(Ns, count, K);
+    if (!workspace || (uintptr_t)workspace % 16) split = 1;
+    while (split > 1 && workspace_bytes < split * outs * 4) split--;
+    // short grids pay only when split
+    if (lists && (split > 1 || blocks >= kGemvTallRows)) {
+      a.split = split;
+      float* p = (float*)workspace;
+      for (int i = 0; i < count && split > 1; i++) {
+        a.mat[i].part = p;
+        p += (size_t)split * M * Ns[i];
+      }
+      return aq::check_hip(launch_qlinear_mid(a, fmt, per_channel ? 1 : chunk_scales(a) ? 2 : 0, pair, s),
+                           "aq_qlinear: mid launch");
+    }
+  }
   // From M = 2 the shared-x GEMV also takes tall groups with block-wise
   // scales (block-128 gate+up at M = 4: 29.9 against 26.7 us; shorter grids
   // and per-channel scales stay faster re-reading x per tile row below)
@@ -2166,10 +2201,23 @@ extern "C" int aq_qlinear_decode(const void* x, int64_t M, int64_t K, int fmt, i
                                  const void* const* biases, void* const* ys, int prologue, const void* x2,
                                  const void* norm_weight, const void* norm_bias, float eps,
                                  const void* const* residuals, const int32_t* relu, void* stream) {
+  return aq_qlinear_decode_ws(x, M, K, fmt, count, Ns, codes, scales, Gs, row_ptrs, cols, vals, tile_ptrs, tile_ents,
+                              biases, ys, prologue, x2, norm_weight, norm_bias, eps, residuals, relu, nullptr, 0,
+                              stream);
+}
+
+extern "C" int aq_qlinear_decode_ws(const void* x, int64_t M, int64_t K, int fmt, int64_t count, const int64_t* Ns,
+                                    const void* const* codes, const void* const* scales, const int64_t* Gs,
+                                    const int32_t* const* row_ptrs, const int32_t* const* cols,
+                                    const void* const* vals, const int32_t* const* tile_ptrs,
+                                    const uint32_t* const* tile_ents, const void* const* biases, void* const* ys,
+                                    int prologue, const void* x2, const void* norm_weight, const void* norm_bias,
+                                    float eps, const void* const* residuals, const int32_t* relu, void* workspace,
+                                    int64_t workspace_bytes, void* stream) {
   const DecodeFuse fz{prologue, x2, norm_weight, norm_bias, eps, residuals, relu};
   // no tile_max: the decode GEMVs never take the GEMM
   return qlinear_grouped_impl(x, M, K, fmt, count, Ns, codes, scales, Gs, row_ptrs, cols, vals, tile_ptrs, tile_ents,
-                              nullptr, biases, ys, nullptr, 0, stream, &fz);
+                              nullptr, biases, ys, workspace, workspace_bytes, stream, &fz);
 }
 
 extern "C" int aq_qlinear(const void* x, int64_t M, int64_t K, int64_t N, const void* codes, const void* scales,

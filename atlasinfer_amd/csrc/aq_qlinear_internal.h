@@ -133,4 +133,11 @@ __device__ __forceinline__ uint32_t tile_off(int row, int piece) {
 constexpr uint32_t kOutOfRange = 0x80000000u;  // a buffer offset past every range used here
 constexpr int kBufferDword3 = 0x00020000;      // raw (untyped) buffer access on gfx9
 
+// aq_qlinear_mid.hip: the linear for kMidMinM..kMidMaxM rows of x, a.split
+// parts of K (partial sums at a.mat[i].part when more than one); pc: the
+// scale mode of the GEMVs.  mid_split: the parts a launch wants.
+constexpr int kMidMinM = 33, kMidMaxM = 64;
+int mid_split(const int64_t* Ns, int64_t count, int64_t K);
+hipError_t launch_qlinear_mid(QLArgs a, int fmt, int pc, bool pair, hipStream_t s);
+
 }  // namespace aqk

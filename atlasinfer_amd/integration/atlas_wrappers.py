@@ -148,13 +148,16 @@ def qlinear_decode(x: torch.Tensor, qts, biases, codes, prologue: int = PRO_NONE
         tps, tes = arr([t[0].data_ptr() for t in tiles]), arr([t[1].data_ptr() for t in tiles])
     else:
         tps = tes = None
-    _lib.check(L.aq_qlinear_decode(
+    ws_bytes = int(L.aq_qlinear_decode_workspace_size(M, sum(Ns), K)) if M >= GEMM_MIN_M else 0
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
+    _lib.check(L.aq_qlinear_decode_ws(
         xs[0].data_ptr(), M, K, _format_id(fmt), n, arr(Ns, ctypes.c_int64), arr([c.data_ptr() for c in codes]),
         arr([q.scale_factors.data_ptr() for q in qts]), arr([q.block_size for q in qts], ctypes.c_int64),
         arr([q.outlier_row_ptr.data_ptr() for q in qts]), arr([_lib.ptr(q.outlier_cols) for q in qts]),
         arr([_lib.ptr(q.fp16_outliers) for q in qts]), tps, tes, arr([_lib.ptr(b) for b in biases]),
         arr(yp), int(prologue), None if x2 is None else xs[1].data_ptr(), _lib.ptr(norm_weight),
-        _lib.ptr(norm_bias), ctypes.c_float(eps), res, acts, _lib.stream_of(dev)), "aq_qlinear_decode")
+        _lib.ptr(norm_bias), ctypes.c_float(eps), res, acts, _lib.ptr(ws), ws_bytes, _lib.stream_of(dev)),
+        "aq_qlinear_decode_ws")
     return ys
 
 

@@ -340,6 +340,21 @@ int aq_qlinear_decode(const void* x, int64_t M, int64_t K, int fmt, int64_t coun
                       float eps, const void* const* residuals, const int32_t* relu, void* stream);
 
 /*
+ * aq_qlinear_decode with a workspace, as aq_qlinear_grouped's: with
+ * aq_qlinear_decode_workspace_size(M, sum of Ns, K) bytes (0 for most calls),
+ * calls of 33 to 64 rows with the block lists split K over workgroups and keep
+ * the fp32 partial sums there (NULL, or less: a smaller split, or none).
+ */
+int64_t aq_qlinear_decode_workspace_size(int64_t M, int64_t N, int64_t K);
+int aq_qlinear_decode_ws(const void* x, int64_t M, int64_t K, int fmt, int64_t count, const int64_t* Ns,
+                         const void* const* codes, const void* const* scales, const int64_t* Gs,
+                         const int32_t* const* row_ptrs, const int32_t* const* cols, const void* const* vals,
+                         const int32_t* const* tile_ptrs, const uint32_t* const* tile_ents, const void* const* biases,
+                         void* const* ys, int prologue, const void* x2, const void* norm_weight, const void* norm_bias,
+                         float eps, const void* const* residuals, const int32_t* relu, void* workspace,
+                         int64_t workspace_bytes, void* stream);
+
+/*
  * Attention of one decode step over a static key/value cache, the position
  * read from device memory (so that a captured HIP graph replays it for
  * every token).  Replaces the attention part of a decode step's forward:

@@ -1,0 +1,107 @@
+"""qlinear_decode at 33 to 64 rows, where short and tall grids split K over
+workgroups: against the float64 product of x and the dequantized weight, with
+every split the workspace allows (the parts' sums differ in order only), the
+decode epilogue, ragged last units, odd part lengths and crowded blocks."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from atlasinfer_amd import _lib
+from atlasinfer_amd.integration import atlas_wrappers as AW
+from atlasinfer_amd.quant import adaptive_quantizer as AQ
+from gpu_ref import make_weights
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda", 0)
+
+
+def _weight(N, K, G, fmt, seed, frac=0.002, thr=3.0):
+    rng = np.random.default_rng(seed)
+    w = torch.from_numpy(make_weights(rng, (N, K), t_dof=3, frac=frac)).to(DEV)
+    q = AQ.quantize_tensor(w, G, thr, code_format=fmt)
+    deq = AQ.dequantize_tensor(q, DEV).double()
+    AQ.discard_dequantized(id(q))
+    return q, deq
+
+
+def _x(M, K, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return torch.randn(M, K, generator=g, device=DEV).half()
+
+
+def _close(y, x, deq, bias=None):
+    want = x.double() @ deq.t()
+    if bias is not None:
+        want = want + bias.double()
+    ulp = torch.from_numpy(np.spacing(np.abs(want.cpu().numpy()).astype(np.float16)).astype(np.float64)).to(DEV)
+    # one rounding of the output and a worst-case f32 accumulation error
+    bound = ulp + 2.0 ** -20 * (x.double().abs() @ deq.abs().t())
+    assert ((y.double() - want).abs() <= bound).all()
+
+
+# rows, cols, block, rows of x, format: units of 128 columns that end inside
+# the matrix (48, 272), chunks that do not divide by the parts (7, 11, 23),
+# scales per row, per chunk and finer, both row-group counts
+@pytest.mark.parametrize("N,K,G,M,fmt", [(48, 896, -1, 33, "e4m3"), (272, 1408, 128, 48, "e4m3"),
+                                         (4096, 2944, 64, 49, "e4m3"), (1024, 4096, 256, 64, "int8"),
+                                         (256, 9472, -1, 64, "e4m3"), (12304, 1024, -1, 40, "e4m3")])
+def test_mid_matches_dequantized_product(N, K, G, M, fmt):
+    q, deq = _weight(N, K, G, fmt, N + K)
+    x = _x(M, K, M)
+    bias = _x(1, N, 5)[0]
+    res = _x(M, N, 6)
+    codes, tiles = [AQ.kernel_codes(q, DEV)], [AQ.outlier_tiles(q, DEV)]
+    y = AW.qlinear_decode(x, [q], [bias], codes, tiles=tiles)[0]
+    _close(y, x, deq, bias)
+    z = AW.qlinear_decode(x, [q], [bias], codes, tiles=tiles, relu=[1], residuals=[res])[0]
+    assert torch.equal(z, torch.relu(y) + res)
+    assert torch.equal(y, AW.qlinear_decode(x, [q], [bias], codes, tiles=tiles)[0])  # deterministic
+
+
+def test_mid_every_split():
+    """A workspace of s parts' bytes, less one, or none: fewer parts, same result to f32 rounding."""
+    N, K, M = 512, 3200, 64
+    q, deq = _weight(N, K, 128, "e4m3", 3)
+    x = _x(M, K, 1)
+    L, arr = _lib.load(), _lib.ptr_array
+    tp, te, _ = AQ.outlier_tiles(q, DEV)
+    full = int(L.aq_qlinear_decode_workspace_size(M, N, K))
+    assert full >= 2 * M * N * 4 and full % (M * N * 4) == 0
+    for nbytes in [0] + [p * M * N * 4 - 16 * (p % 2) for p in range(1, full // (M * N * 4) + 1)]:
+        ws = torch.full((max(nbytes, 16),), 0xFF, dtype=torch.uint8, device=DEV)  # NaN where nothing is written
+        y = torch.empty(M, N, dtype=torch.float16, device=DEV)
+        _lib.check(L.aq_qlinear_decode_ws(
+            x.data_ptr(), M, K, _lib.FMT_E4M3, 1, arr([N], ctypes.c_int64), arr([q.fp8_data.data_ptr()]),
+            arr([q.scale_factors.data_ptr()]), arr([q.block_size], ctypes.c_int64), arr([q.outlier_row_ptr.data_ptr()]),
+            arr([q.outlier_cols.data_ptr()]), arr([q.fp16_outliers.data_ptr()]), arr([tp.data_ptr()]),
+            arr([te.data_ptr()]), arr([None]), arr([y.data_ptr()]), 0, None, None, None, ctypes.c_float(0), None, None,
+            ws.data_ptr() if nbytes else None, nbytes, _lib.stream_of(DEV)), "aq_qlinear_decode_ws")
+        _close(y, x, deq)
+
+
+def test_mid_grouped_and_swiglu_pair():
+    """Members of different sizes in one launch; gate and up as a pair, split and not."""
+    K, M = 1664, 50
+    ws = [_weight(n, K, -1, "e4m3", n) for n in (1040, 256, 16)]
+    x = _x(M, K, 2)
+    ys = AW.qlinear_decode(x, [w[0] for w in ws], [None] * 3, [w[0].fp8_data.view(torch.uint8) for w in ws])
+    for y, (_, deq) in zip(ys, ws):
+        _close(y, x, deq)
+    for N in (80, 1616, 8208):
+        (g, dg), (u, du) = _weight(N, K, 128, "e4m3", 1), _weight(N, K, 128, "e4m3", 2)
+        codes = [q.fp8_data.view(torch.uint8) for q in (g, u)]
+        a = AW.qlinear_decode(x, [g, u], [None, None], codes, swiglu_pair=True)[0]
+        yg, yu = AW.qlinear_decode(x, [g, u], [None, None], codes)
+        want = torch.nn.functional.silu(yg.float()).half() * yu
+        assert (a.float() - want.float()).abs().max() <= 2.0 ** -9 * want.float().abs().max()
+
+
+def test_mid_crowded_blocks():
+    """Chunks with more outliers than travel with the codes (8), and more than 64."""
+    q, deq = _weight(64, 1024, 128, "e4m3", 9, frac=0.05, thr=1.2)
+    assert int(q.outlier_tile_max) > 64
+    x = _x(64, 1024, 4)
+    y = AW.qlinear_decode(x, [q], [None], [q.fp8_data.view(torch.uint8)])[0]
+    _close(y, x, deq)
