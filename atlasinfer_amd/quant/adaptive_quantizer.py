@@ -34,6 +34,7 @@ Code formats:
 from __future__ import annotations
 
 import ctypes
+import functools
 import threading
 from typing import NamedTuple, Optional
 
@@ -264,6 +265,7 @@ def quantize_tensor(
     p = _quantize_prepare(fp16_tensor, G, z_threshold, code_format, fmt)
     L = _lib.load()
     _lib.check(L.aq_quantize(*p["args"], p["stream"]), "aq_quantize")
+    _queue_behind(p)
     nnz = int(p["block_off"][p["nblocks"]].item())  # the one host sync: sizes the outlier tensors
     return _quantize_complete(p, nnz)
 
@@ -297,25 +299,45 @@ def _a256(n: int) -> int:
     return (n + 255) // 256 * 256
 
 
+class _ShapePlan(NamedTuple):
+    """What a weight's quantize needs that follows from its shape, block size
+    and format alone."""
+    numel: int
+    N: int
+    K: int
+    nblocks: int
+    padded: int
+    layout: str
+    ws_bytes: int  # workspace, a multiple of 256
+    ntile: int     # block-list pointers (tiled layout)
+    sizes: tuple   # bytes of codes, scales, block offsets, block-list pointers, multiples of 256
+
+
+@functools.lru_cache(maxsize=4096)
+def _shape_plan(shape: torch.Size, G: int, fmt: int) -> _ShapePlan:
+    N, K = _rows_cols(shape)
+    numel = N * K
+    nblocks = (numel + G - 1) // G
+    layout = _layout_of(fmt, shape, G)
+    ntile = (N // 16) * (K // 64) + 1 if layout == "tiled" else 0
+    return _ShapePlan(numel, N, K, nblocks, nblocks * G, layout,
+                      _a256(int(_lib.load().aq_quantize_workspace_size(numel, G))), ntile,
+                      tuple(_a256(nb) for nb in (nblocks * G, 2 * nblocks, 4 * (nblocks + 1), 4 * ntile)))
+
+
 def _run_plan(tensors, G: int, fmt: int, code_format: str, dev: torch.device):
     """The members of a tiled run before anything is allocated for them, and
     the byte offsets of their codes, scales, block offsets and block-list
     pointers in one buffer for the run (each 256-byte aligned)."""
     ps, at = [], 0
     for t in tensors:
-        numel = t.numel()
         x = t if t.device == dev and t.is_contiguous() else t.to(dev).contiguous()
-        N, K = _rows_cols(t.shape)
-        nblocks = (numel + G - 1) // G
-        ntile = (N // 16) * (K // 64) + 1
-        p = dict(x=x, input_device=t.device, original_shape=t.shape, numel=numel, G=G, N=N, K=K, nblocks=nblocks,
-                 padded=nblocks * G, ntile=ntile, layout="tiled", fmt=fmt, code_format=code_format, dev=dev)
-        offs = []
-        for nb in (nblocks * G, 2 * nblocks, 4 * (nblocks + 1), 4 * ntile):  # codes, scales, offsets, pointers
-            offs.append(at)
-            at += _a256(nb)
-        p["at"] = tuple(offs)
-        ps.append(p)
+        w = _shape_plan(t.shape, G, fmt)
+        c, s, o, e = w.sizes
+        ps.append(dict(x=x, input_device=t.device, original_shape=t.shape, numel=w.numel, G=G, N=w.N, K=w.K,
+                       nblocks=w.nblocks, padded=w.padded, ntile=w.ntile, layout="tiled", fmt=fmt,
+                       code_format=code_format, dev=dev, at=(at, at + c, at + c + s, at + c + s + o)))
+        at += c + s + o + e
     return ps, at
 
 
@@ -355,6 +377,21 @@ def _quantize_prepare(fp16_tensor: torch.Tensor, G: int, z_threshold: float, cod
     return p
 
 
+def _queue_behind(p: dict) -> None:
+    """What the result needs besides the outlier lists and does not depend on
+    their length, queued while the quantize kernel runs instead of after the
+    wait for the outlier count: the CSR row pointers and the zeroed word for
+    the largest block count."""
+    if p["K"] % p["G"] == 0:
+        # blocks tile the rows, so a row's first outlier is its first block's:
+        # the row pointers are every (K / G)-th block offset (per output
+        # channel, the block offsets themselves)
+        step = p["K"] // p["G"]
+        p["row_ptr"] = p["block_off"] if step == 1 else p["block_off"][::step].contiguous()
+    if p["layout"] == "tiled" and "tmax" not in p:
+        p["tmax"] = torch.zeros(1, dtype=torch.int32, device=p["dev"])
+
+
 def _finish_outputs(p: dict, nnz: int):
     """The outlier list tensors of a tensor with ``nnz`` outliers (flat
     indices, values, columns) and, for the tiled layout, its block-list
@@ -373,13 +410,9 @@ def _finished_tensor(p: dict, nnz: int, flat_idx, vals, cols, tile_ent, tmax: Op
     block count of the tiled layout's lists (read when first used)."""
     L = _lib.load()
     dev, G, K, N = p["dev"], p["G"], p["K"], p["N"]
-    block_off, codes, padded = p["block_off"], p["codes"], p["padded"]
-    if K % G == 0:
-        # blocks tile the rows, so a row's first outlier is its first block's:
-        # the CSR row pointers are every (K / G)-th block offset (per output
-        # channel, the block offsets themselves)
-        row_ptr = block_off if G == K else block_off[::K // G].contiguous()
-    else:
+    codes, padded = p["codes"], p["padded"]
+    row_ptr = p.get("row_ptr")  # _queue_behind
+    if row_ptr is None:
         row_ptr = torch.empty(N + 1, dtype=torch.int32, device=dev)
         _lib.check(L.aq_segment_offsets(_lib.ptr(flat_idx), nnz, N, K, row_ptr.data_ptr(), p["stream"]),
                    "aq_segment_offsets")
@@ -421,7 +454,7 @@ def _quantize_complete(p: dict, nnz: int) -> QuantizedTensor:
             _lib.ptr(flat_idx), _lib.ptr(vals), _lib.ptr(cols))
     tmax = None
     if tile_ent is not None:
-        t = torch.zeros(1, dtype=torch.int32, device=p["dev"])
+        t = p["tmax"]
         _lib.check(L.aq_quantize_finish_tiles(*args, p["tile_ptr"].data_ptr(), tile_ent.data_ptr(), t.data_ptr(),
                                               p["stream"]), "aq_quantize_finish_tiles")
         tmax = DeviceInt(t, 0)
@@ -458,16 +491,16 @@ def _run_launch(tensors, key, z_bits: int, fmt: int, code_format: str) -> dict:
         ps = [_member_prepare(t, G, fmt, code_format, layout, dev) for t in tensors]
         addr = [(p["codes"].data_ptr(), p["scales"].data_ptr(), p["block_off"].data_ptr(), None) for p in ps]
     n = len(ps)
-    ws_bytes = [(int(L.aq_quantize_workspace_size(p["numel"], G)) + 255) // 256 * 256 for p in ps]
+    ws_bytes = [_shape_plan(p["original_shape"], G, fmt).ws_bytes for p in ps]
     ws = torch.empty(sum(ws_bytes), dtype=torch.uint8, device=dev)
     ws_ptrs, at = [], ws.data_ptr()
     for b in ws_bytes:
         ws_ptrs.append(at)
         at += b
-    # [0, n): the outlier counts; [n, 2n): the block lists' largest counts,
-    # raised from 0 by the finish
-    aux = torch.zeros(2 * n, dtype=torch.int32, device=dev) if layout == "tiled" else \
-        torch.empty(n, dtype=torch.int32, device=dev)
+    # [0, n): the outlier counts, written by the scan; [n, 2n): the block
+    # lists' largest counts, raised from 0 by the finish (zeroed behind the
+    # launch)
+    aux = torch.empty(2 * n if layout == "tiled" else n, dtype=torch.int32, device=dev)
     stream = _lib.stream_of(dev)
     numels = arr([p["numel"] for p in ps], ctypes.c_int64)
     offs = arr([a[2] for a in addr])
@@ -476,16 +509,22 @@ def _run_launch(tensors, key, z_bits: int, fmt: int, code_format: str) -> dict:
         n, arr([p["x"].data_ptr() for p in ps]), numels, G, z_bits, fmt, K, _lib.LAYOUTS[layout],
         arr([a[0] for a in addr]), arr([a[1] for a in addr]), offs, ws_ptrs, ws_bytes, aux.data_ptr(), stream),
         "aq_quantize_grouped")
-    counts = torch.empty(aux.numel(), dtype=torch.int32, pin_memory=True)
-    counts.copy_(aux, non_blocking=True)
+    counts = torch.empty(n, dtype=torch.int32, pin_memory=True)
+    counts.copy_(aux[:n], non_blocking=True)
     done = torch.cuda.Event()
     done.record(torch.cuda.current_stream(dev))
+    tile_ptrs = None
     if buf is not None:
+        aux[n:].zero_()
         _run_views(ps, buf)
+        tile_ptrs = arr([a[3] for a in addr])
     for p, w, b in zip(ps, ws_ptrs, ws_bytes):
         p["ws_ptr"], p["ws_bytes"], p["stream"] = w, b, stream
+        if buf is not None:
+            p["tmax"] = aux
+        _queue_behind(p)
     return dict(ps=ps, ws=ws, aux=aux, counts=counts, done=done, stream=stream, G=G, K=K, numels=numels, offs=offs,
-                ws_ptrs=ws_ptrs, ws_bytes=ws_bytes)
+                ws_ptrs=ws_ptrs, ws_bytes=ws_bytes, tile_ptrs=tile_ptrs)
 
 
 def _run_complete(r: dict) -> list:
@@ -496,7 +535,7 @@ def _run_complete(r: dict) -> list:
     ps = r["ps"]
     n = len(ps)
     r["done"].synchronize()
-    nnzs = r["counts"].tolist()[:n]
+    nnzs = r["counts"].tolist()
     if ps[0]["layout"] != "tiled":
         return [_quantize_complete(p, nnz) for p, nnz in zip(ps, nnzs)]
     L = _lib.load()
@@ -518,7 +557,7 @@ def _run_complete(r: dict) -> list:
     _lib.check(L.aq_quantize_finish_tiles_grouped(
         n, r["numels"], r["G"], r["K"], r["offs"], arr(nnzs, ctypes.c_int64), r["ws_ptrs"], r["ws_bytes"],
         arr([nz(sp[0], k) for sp, k in zip(spans, nnzs)]), arr([nz(sp[1], k) for sp, k in zip(spans, nnzs)]),
-        arr([nz(sp[2], k) for sp, k in zip(spans, nnzs)]), arr([p["tile_ptr"].data_ptr() for p in ps]),
+        arr([nz(sp[2], k) for sp, k in zip(spans, nnzs)]), r["tile_ptrs"],
         arr([b0 + sp[3] for sp in spans]), aux.data_ptr() + 4 * n, r["stream"]), "aq_quantize_finish_tiles_grouped")
     r["ws"] = None  # the finish is queued: the workspace may go back to the allocator
     i64, f16, i32 = lists.view(torch.int64), lists.view(torch.float16), lists.view(torch.int32)
@@ -557,7 +596,8 @@ def quantize_tensors(tensors, block_size: int = 128, z_threshold: float = 3.0, *
             L = _lib.load()
         if G > L.aq_max_block_size():
             raise ValueError(f"block_size {G} exceeds the supported maximum {L.aq_max_block_size()}")
-        key = (_lib.compute_device(t.device), G, _rows_cols(t.shape)[1], _layout_of(fmt, t.shape, G))
+        w = _shape_plan(t.shape, G, fmt)
+        key = (_lib.compute_device(t.device), G, w.K, w.layout)
         groups.setdefault(key, []).append(i)
     runs = []
     for key, idx in groups.items():
