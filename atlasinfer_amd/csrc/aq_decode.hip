@@ -301,7 +301,9 @@ __global__ __launch_bounds__(64 * kMaxWaves) void decode_attention_kernel(
       const float sg = valid ? (float)rn_h(dot) * scale : -INFINITY;
       mn[g] = fmaxf(m[g], max4<KV>(sg));  // the same in every lane of a row group
       grows = grows || mn[g] != m[g];
-      e[g] = valid ? __expf(sg - mn[g]) : 0.0f;
+      // a score of -inf (an fp16 overflow) weighs nothing, also while its row
+      // group has met no other
+      e[g] = sg == -INFINITY ? 0.0f : __expf(sg - mn[g]);
     }
     if (__ballot(grows)) {
 #pragma unroll

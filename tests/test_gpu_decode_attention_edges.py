@@ -62,3 +62,34 @@ def test_one_and_few_spans(D, G, pos):
 ])
 def test_long_caches(B, Hkv, G, D, L, pos):
     _run(B, Hkv, G, D, L, pos, pos)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("pos,low", [(40, 32), (700, 650), (4000, 64)])
+def test_scores_of_minus_infinity(D, pos, low):
+    """The first ``low`` positions' scores overflow fp16 to -inf, for whole
+    steps, waves and spans: they weigh nothing, and the rest come out as if
+    alone."""
+    Hkv, L = 2, 4160
+    g = torch.Generator(device=DEV).manual_seed(pos + D)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV).half()  # noqa: E731
+    q = rnd(1, Hkv, D).abs() + 1.0
+    kc, vc, k, v = rnd(1, Hkv, L, D) * 0.1, rnd(1, Hkv, L, D), rnd(1, Hkv, D) * 0.1, rnd(1, Hkv, D)
+    kc[:, :, :low] = -60000.0  # products below -60000 D
+    Lb = _lib.load()
+    nb = Lb.aq_decode_attention_workspace(1, Hkv, Hkv, D, L)
+    ws = torch.full((max(nb, 16),), 0xFF, dtype=torch.uint8, device=DEV)
+    out = torch.empty(1, Hkv, D, dtype=torch.float16, device=DEV)
+    p = torch.full((1,), pos, dtype=torch.long, device=DEV)
+    scale = D ** -0.5
+    _lib.check(Lb.aq_decode_attention(q.data_ptr(), k.data_ptr(), v.data_ptr(), kc.data_ptr(), vc.data_ptr(),
+                                      p.data_ptr(), 1, Hkv, Hkv, D, L, ctypes.c_float(scale), ctypes.c_float(1.0), None,
+                                      None, ws.data_ptr(), nb, out.data_ptr(), _lib.stream_of(DEV)), "attention")
+    s = (kc[:, :, low:pos + 1].double() * q.double().unsqueeze(2)).sum(-1)
+    vv = vc[:, :, low:pos + 1].double()
+    w = torch.softmax(s * scale, -1)
+    want = (vv * w.unsqueeze(-1)).sum(2)
+    # as in _run
+    off = (s.abs().amax(-1) * scale * 2.0 ** -11 * 2 + 2.0 ** -10).unsqueeze(-1)
+    bound = off * (vv.abs() * w.unsqueeze(-1)).sum(2) + 2.0 ** -11 * want.abs() + 1e-6
+    assert ((out.double() - want).abs() <= bound).all()
