@@ -87,8 +87,9 @@ struct SpanOutliers {
     const int64_t lb0 = lb[0];
     const int cnt = (int)(lb[1] - lb0);
     for (int i = t; i < cnt; i += 256) {
-      const int e = (int)(idx[lb0 + i] - t0);
-      atomicOr(&bits[e >> 5], 1u << (e & 31));
+      const int64_t e = idx[lb0 + i] - t0;
+      // always so in an ascending list; one that is not writes nothing past bits
+      if ((uint64_t)e < (uint64_t)kSpan) atomicOr(&bits[e >> 5], 1u << (e & 31));
     }
     __syncthreads();
     int total;
