@@ -1962,24 +1962,49 @@ hipError_t launch_gemm_wide(const QLArgs& a, int fmt, bool per_channel, bool den
                             : launch_gemm_wide<AQ_FMT_INT8, 0>(a, per_channel, ws, ws_bytes, s);
 }
 
+// Whether 33 to 64 rows of x on a grid of `blocks` tile rows go to the linear
+// split over K (aq_qlinear_mid.hip), given the block lists and a workspace.
+// Short grids (below 384 tile rows) do: at M = 64 in a decode step o_proj
+// 25 -> 18.4 us and down_proj 90 -> 31 against the shared-x GEMV; against the
+// GEMM, which plain calls took, on up to 256 tile rows [4096, 14336] 33.5 ->
+// 27.9 at M = 33 and 33.2 -> 31.1 at 64, in blocks of 128 36.3 -> 27.6 and
+// 36.6 -> 31.9, [2048, 8192] 22.4 -> 18.3 and 23.0 -> 21.0, [4096, 4096]
+// 16.5 -> 15.9 and 18.5 -> 18.3 ([6000, 4096], 375 tile rows, 23.4 -> 25.9:
+// the GEMM's).  Plain calls of 49 rows or more with K below 4096 stay with it
+// ([2048, 2048] at M = 64 14.4 against 15.1), and weights of heavy tails
+// (1.4 % outliers, up to 35 in a block: [4096, 14336] at M = 64 35.1 against
+// 53.6; the shared-x GEMV, which decode steps had, 84).  Decode steps also
+// take it on tall grids (gate+up
+// 54.5 -> 47 at M = 64; a plain call there has no workspace, and unsplit it
+// gains nothing); between the two the shared-x GEMV stays ahead (q/k/v 22.3
+// against 24.5, [8192, 2048] 14.6 against 19).  Two bands of up to 64 rows did
+// not carry it past 64: [8192, 2048] at M = 128 24.7 us against the GEMM's
+// 22.7, [4096, 14336] 44.9 against 36.2.
+bool mid_takes(int64_t M, int64_t blocks, int64_t K, bool decode) {
+  if (M < kMidMinM || M > kMidMaxM) return false;
+  if (decode) return blocks < kGemvShortRows || blocks >= kGemvTallRows;
+  return blocks <= kMidPlainMaxRows && (M <= kMidPlainMaxM || K >= kMidPlainMinK);
+}
+
 }  // namespace
 
 extern "C" int64_t aq_qlinear_workspace_size(int64_t M, int64_t N, int64_t K) {
   // the GEMM's fp32 partial sums when it would split K for this shape on the
   // current device (0 for the GEMV and for unsplit grids; for 33 <= M <= 64
-  // on short grids the GEMM takes the call if given the block lists)
+  // on short grids the split-K linear or the GEMM takes the call if given the block lists)
   if (N <= 0 || K < 128 || K % 128) return 0;
   if (M <= kGemvShortMaxM || (M <= kGemvMaxM && N / 16 >= kGemvShortRows)) return 0;
   const GemmPlan p = plan_gemm(M, &N, 1, K, 8);
-  if (p.split > 1) return p.split * M * N * 4;
+  // the larger of the two, as the split-K linear may leave the call to the GEMM
+  const int split = std::max(p.split, mid_takes(M, N / 16, K, false) ? mid_split(&N, 1, K) : 1);
+  if (split > 1) return split * M * N * 4;
   int64_t tail_bytes = 0;  // an unsplit 256 x 256 grid's tail tiles, run as two K halves
   if (p.tile == kTile256x256) wide_tail(aq::ceil_div(N, kWideBN) * aq::ceil_div(M, kWideBM), K, &tail_bytes);
   return tail_bytes;
 }
 
 extern "C" int64_t aq_qlinear_decode_workspace_size(int64_t M, int64_t N, int64_t K) {
-  if (N <= 0 || K < 128 || K % 128 || M < kMidMinM || M > kMidMaxM) return 0;
-  if (N / 16 >= kGemvShortRows && N / 16 < kGemvTallRows) return 0;
+  if (N <= 0 || K < 128 || K % 128 || !mid_takes(M, N / 16, K, true)) return 0;
   const int split = mid_split(&N, 1, K);
   return split > 1 ? split * M * N * 4 : 0;
 }
@@ -2094,13 +2119,11 @@ static int qlinear_grouped_impl(const void* x, int64_t M, int64_t K, int fmt, in
   bool have_lists = tile_ptrs && tile_ents && tile_maxes;
   for (int i = 0; i < count && have_lists; i++) have_lists = tile_ptrs[i] && tile_ents[i];
   const bool gemv = M <= kGemvShortMaxM || (M <= kGemvMaxM && (blocks >= kGemvShortRows || !have_lists));
-  // Decode steps of 33 rows of x or more, given the block lists: short grids
-  // (below 384 tile rows) and tall ones (768 or more) split K over workgroups (aq_qlinear_mid.hip): at M = 64
-  // o_proj 25 -> 18.4 us and down_proj 90 -> 31 in a decode step, gate+up
-  // 54.5 -> 47.  Between them the shared-x GEMV stays ahead (q/k/v 22.3
-  // against 24.5, [8192, 2048] 14.6 against 19).
-  if (fz && M >= kMidMinM && M <= kMidMaxM && (blocks < kGemvShortRows || blocks >= kGemvTallRows) &&
-      tile_ptrs && tile_ents) {
+  bool mid = mid_takes(M, blocks, K, fz != nullptr) && tile_ptrs && tile_ents;
+  // more outliers than that in a block take rounds of their own, in which
+  // nothing is in flight; decode calls don't know the count
+  for (int i = 0; i < count && mid && !fz; i++) mid = tile_maxes && tile_maxes[i] <= kMidPlainMaxOutl;
+  if (mid) {
     const bool pair = a.mat[0].act == 2;
     bool lists = true;
     int64_t outs = 0;

@@ -257,7 +257,8 @@ int aq_zscore(const void* x, int64_t n, float eps, void* z, void* stats, void* s
  * accumulated in fp32, plus the bias, rounded once to fp16.
  * workspace: aq_qlinear_workspace_size(M, N, K) bytes, 16-byte aligned, or
  * NULL.  A nonzero size means the GEMM would split K (2, 4 or 8 ways, chosen
- * from a time estimate of the shape on the current device) and keep the fp32
+ * from a time estimate of the shape on the current device), or 33 to 64 rows
+ * on a short grid would (up to 16 ways), and keep the fp32
  * partial sums there; a second kernel adds them in a fixed order, so results
  * are deterministic.  A smaller workspace, or NULL, only limits the split (to
  * what it holds, down to none).  0 for every GEMV call.

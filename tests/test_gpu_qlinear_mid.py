@@ -105,3 +105,48 @@ def test_mid_crowded_blocks():
     x = _x(64, 1024, 4)
     y = AW.qlinear_decode(x, [q], [None], [q.fp8_data.view(torch.uint8)])[0]
     _close(y, x, deq)
+
+
+# plain linears on both sides of the rule (more than 48 rows with K below 4096
+# and weights with more than 20 outliers in a block take the GEMM), ragged last
+# units, all scale modes
+@pytest.mark.parametrize("thr", [3.0, 8.0])
+@pytest.mark.parametrize("M", [33, 48, 49, 64])
+@pytest.mark.parametrize("N,K,G,fmt", [(48, 1024, -1, "e4m3"), (272, 3968, 128, "int8"), (2064, 4096, 64, "e4m3")])
+def test_mid_plain(N, K, G, fmt, M, thr):
+    q, deq = _weight(N, K, G, fmt, N + K, thr=thr)
+    x, bias = _x(M, K, M), _x(1, N, 5)[0]
+    tiles = AQ.outlier_tiles(q, DEV)
+    y = AW.qlinear(x, q, bias, codes=AQ.kernel_codes(q, DEV), tiles=tiles)
+    _close(y, x, deq, bias)
+    if int(tiles[2]) <= 20 and (M <= 48 or K >= 4096):  # the decode call's sums
+        assert torch.equal(y, AW.qlinear_decode(x, [q], [bias], [AQ.kernel_codes(q, DEV)], tiles=[tiles])[0])
+
+
+@pytest.mark.parametrize("M", [33, 48, 64])
+def test_mid_plain_grouped(M):
+    """Members of different sizes in one launch."""
+    K = 1664
+    ws = [_weight(n, K, -1, "e4m3", n, thr=8.0) for n in (1040, 256, 16)]
+    x = _x(M, K, 2)
+    for y, (_, deq) in zip(AW.qlinear_grouped(x, [w[0] for w in ws]), ws):
+        _close(y, x, deq)
+
+
+@pytest.mark.parametrize("parts", [0, 1, 2, 3])
+def test_mid_plain_workspaces(parts):
+    """Workspaces too small for two parts leave the call to the GEMM or the GEMV, others limit the split."""
+    N, K = 512, 3200
+    q, deq = _weight(N, K, 128, "e4m3", 3, thr=8.0)
+    tp, te, tmax = AQ.outlier_tiles(q, DEV)
+    for M in (40, 64):
+        x = _x(M, K, 1)
+        nbytes = parts * M * N * 4
+        ws = torch.full((max(nbytes, 16),), 0xFF, dtype=torch.uint8, device=DEV)  # NaN where nothing is written
+        y = torch.empty(M, N, dtype=torch.float16, device=DEV)
+        _lib.check(_lib.load().aq_qlinear(
+            x.data_ptr(), M, K, N, q.fp8_data.data_ptr(), q.scale_factors.data_ptr(), q.block_size, _lib.FMT_E4M3,
+            q.outlier_row_ptr.data_ptr(), q.outlier_cols.data_ptr(), q.fp16_outliers.data_ptr(), tp.data_ptr(),
+            te.data_ptr(), tmax, None, y.data_ptr(), ws.data_ptr() if nbytes else None, nbytes, _lib.stream_of(DEV)),
+            "aq_qlinear")
+        _close(y, x, deq)
