@@ -88,7 +88,8 @@ struct SpanOutliers {
     const int cnt = (int)(lb[1] - lb0);
     for (int i = t; i < cnt; i += 256) {
       const int64_t e = idx[lb0 + i] - t0;
-      // always so in an ascending list; one that is not writes nothing past bits
+      // always so in an ascending list; one that is not writes nothing past
+      // bits (and may put a run's codes outside the stream: the callers look)
       if ((uint64_t)e < (uint64_t)kSpan) atomicOr(&bits[e >> 5], 1u << (e & 31));
     }
     __syncthreads();
@@ -115,11 +116,15 @@ __device__ __forceinline__ uint64_t load8(const uint8_t* p) {
 }
 __device__ __forceinline__ uint64_t low_bytes(int n) { return ((uint64_t)1 << (8 * n)) - 1; }  // n < 8
 
-// The codes of a run from the compacted stream: 8 - popcount(bits) codes at
-// src (`avail` of them and more behind readable), a 0 code put in at each
-// flagged element.
-__device__ __forceinline__ uint64_t stream_codes(const uint8_t* src, int64_t avail, uint32_t bits, int n) {
+// The codes of a run from a compacted stream of `len` codes: n - popcount(bits)
+// of them from position c0 on, a 0 code put in at each flagged element.
+// Nothing outside the stream is read: c0 is negative after repeated indices.
+__device__ __forceinline__ uint64_t stream_codes(const uint8_t* stream, int64_t len, int64_t c0, uint32_t bits,
+                                                 int n) {
   uint64_t w = 0;
+  if (c0 < 0) return w;
+  const uint8_t* src = stream + c0;
+  const int64_t avail = len - c0;
   if (avail >= 8) {
     w = load8(src);
   } else {
@@ -156,7 +161,7 @@ __global__ __launch_bounds__(256) void reorder_codes_kernel(const uint8_t* src, 
     uint32_t bits = so.run(off, &pre);
     const int64_t c0 = j0 - lb0 - pre;  // the run's first code in the stream
     if (MODE == 1) {
-      uint64_t w = stream_codes(src + c0, padded - nnz - c0, bits, n);
+      uint64_t w = stream_codes(src, padded - nnz, c0, bits, n);
       if (n == 8) {
         __builtin_memcpy(dst + j0, &w, 8);
       } else {
@@ -171,6 +176,7 @@ __global__ __launch_bounds__(256) void reorder_codes_kernel(const uint8_t* src, 
         bits &= (1u << n) - 1u;
       }
       const int left = n - __builtin_popcount(bits);
+      if (c0 < 0 || c0 + left > padded - nnz) continue;  // only after indices that do not ascend
       while (bits) {  // from the last flagged element down
         const int e = 31 - __builtin_clz(bits);
         bits &= ~(1u << e);
@@ -305,7 +311,7 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* codes, cons
     if (STREAM) {
       bits = so.run(off, &pre);
       const int64_t c0 = j0 - lb0 - pre;
-      w = stream_codes(codes + c0, padded - nnz - c0, bits, (int)min((int64_t)8, padded - j0));
+      w = stream_codes(codes, padded - nnz, c0, bits, (int)min((int64_t)8, padded - j0));
     } else if (n == 8) {
       w = load8(codes + j0);
     } else {

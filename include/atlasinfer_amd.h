@@ -190,6 +190,8 @@ int aq_quantize_finish_tiles_grouped(int64_t count, const int64_t* numels, int64
  * read back at :209-212).
  *   aq_compact_codes: dense[padded] -> compact[padded - nnz]
  *   aq_expand_codes:  compact[padded - nnz] -> dense[padded] (0 at outliers)
+ * flat_idx ascending without repeats; after any other list the codes are
+ * undefined, but nothing outside the two buffers is read or written.
  */
 int aq_compact_codes(const void* dense, int64_t padded, const int64_t* flat_idx, int64_t nnz,
                      void* compact, void* stream);

@@ -107,3 +107,37 @@ def test_dequantize_tiled(rows, cols, G, fmt):
         _call("aq_dequantize", tiled.data_ptr(), dsc.data_ptr(), numel, G, fmt, cols, _lib.LAYOUT_TILED,
               _lib.ptr(didx), _lib.ptr(dvals), int(inside.sum()), y.data_ptr() + 2 * shift)
         assert np.array_equal(y.cpu().numpy()[shift:shift + numel].view(np.uint16), want.view(np.uint16))
+
+
+def _lists(padded):
+    """Index lists that do not ascend: repeats, descending, shuffled, past either end."""
+    rng = np.random.default_rng(padded)
+    n = padded // 2
+    return [np.full(n, 5), np.arange(n)[::-1], rng.permutation(padded)[:n], rng.integers(0, padded, n),
+            np.full(n, padded + 99), np.full(n, -3), np.sort(rng.integers(-padded, 2 * padded, n))]
+
+
+@pytest.mark.parametrize("which", range(7))
+@pytest.mark.parametrize("padded", [16384, 24576 + 13])
+def test_lists_that_do_not_ascend_stay_inside(padded, which):
+    """The codes are undefined then, but guards of a list's length on both
+    sides of the buffers are neither written nor read."""
+    idx = np.ascontiguousarray(_lists(padded)[which]).astype(np.int64)
+    nnz, didx = idx.size, _dev(idx)
+    left = padded - nnz
+    dense, stream, y = (torch.full((3 * padded,), 0x5A, dtype=t, device=DEV)
+                        for t in (torch.uint8, torch.uint8, torch.float16))
+    dense[padded:2 * padded] = 7
+    _call("aq_compact_codes", dense[padded:].data_ptr(), padded, didx.data_ptr(), nnz, stream[padded:].data_ptr())
+    assert (stream[:padded] == 0x5A).all() and (stream[padded + left:] == 0x5A).all()
+    stream[padded:padded + left] = 7
+    _call("aq_expand_codes", stream[padded:].data_ptr(), padded, didx.data_ptr(), nnz, dense[padded:].data_ptr())
+    assert (dense[:padded] == 0x5A).all() and (dense[2 * padded:] == 0x5A).all()
+    got = dense[padded:2 * padded]
+    assert ((got == 0) | (got == 7)).all()
+    sc, vals = torch.ones(1, dtype=torch.float16, device=DEV), torch.full((nnz,), 3.0, dtype=torch.float16, device=DEV)
+    _call("aq_dequantize_stream", stream[padded:].data_ptr(), sc.data_ptr(), padded, padded, didx.data_ptr(),
+          vals.data_ptr(), nnz, y[padded:].data_ptr())
+    assert (y[:padded] == 0x5A).all() and (y[2 * padded:] == 0x5A).all()
+    got = y[padded:2 * padded]
+    assert ((got == 0) | (got == 7) | (got == 3)).all()
