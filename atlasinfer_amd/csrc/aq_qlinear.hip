@@ -2005,8 +2005,7 @@ extern "C" int64_t aq_qlinear_workspace_size(int64_t M, int64_t N, int64_t K) {
 
 extern "C" int64_t aq_qlinear_decode_workspace_size(int64_t M, int64_t N, int64_t K) {
   if (N <= 0 || K < 128 || K % 128 || !mid_takes(M, N / 16, K, true)) return 0;
-  const int split = mid_split(&N, 1, K);
-  return split > 1 ? split * M * N * 4 : 0;
+  return mid_split(&N, 1, K) * M * N * 4;
 }
 
 // aq_qlinear_decode's additions to a grouped launch
@@ -2131,14 +2130,14 @@ static int qlinear_grouped_impl(const void* x, int64_t M, int64_t K, int fmt, in
       lists = lists && tile_ptrs[i] && tile_ents[i];
       outs += M * Ns[i];
     }
-    int split = mid_split(Ns, count, K);
-    if (!workspace || (uintptr_t)workspace % 16) split = 1;
-    while (split > 1 && workspace_bytes < split * outs * 4) split--;
+    const int want = mid_split(Ns, count, K);
+    int split = workspace && (uintptr_t)workspace % 16 == 0 ? want : 0;
+    while (split > 0 && workspace_bytes < split * outs * 4) split--;
     // short grids pay only when split
-    if (lists && (split > 1 || blocks >= kGemvTallRows)) {
+    if (lists && (split > 1 || (split == want && blocks >= kGemvTallRows))) {
       a.split = split;
       float* p = (float*)workspace;
-      for (int i = 0; i < count && split > 1; i++) {
+      for (int i = 0; i < count; i++) {
         a.mat[i].part = p;
         p += (size_t)split * M * Ns[i];
       }

@@ -28,7 +28,7 @@ struct QLMat {
   const uint32_t* tent;
   const uint16_t* bias;
   uint16_t* y;
-  float* part;  // GEMM split over K: this matrix's fp32 partial sums [split][M][N]
+  float* part;  // split over K: this matrix's fp32 partial sums [split][M][N]
   int N;       // rows (of a GEMV piece: the rows it covers)
   int G;
   int kg;      // K / G, scale blocks per row
@@ -134,7 +134,7 @@ constexpr uint32_t kOutOfRange = 0x80000000u;  // a buffer offset past every ran
 constexpr int kBufferDword3 = 0x00020000;      // raw (untyped) buffer access on gfx9
 
 // aq_qlinear_mid.hip: the linear for kMidMinM..kMidMaxM rows of x, a.split
-// parts of K (partial sums at a.mat[i].part when more than one); pc: the
+// parts of K (partial sums at a.mat[i].part, also of one part); pc: the
 // scale mode of the GEMVs.  mid_split: the parts a launch wants.
 constexpr int kMidMinM = 33, kMidMaxM = 64;
 // plain calls: up to so many tile rows and outliers in a 16 x 64 block, and so

@@ -16,10 +16,10 @@
 // gathered from LDS against the values).  One barrier a chunk, which waits
 // only for the x of the next chunk.
 //
-// K is split over workgroups until they fill the CUs (mid_split); parts leave
-// fp32 partial sums in the caller's workspace and mid_reduce_kernel adds them
-// in order, with the bias and the decode epilogue.  Unsplit, the epilogue
-// runs here.
+// K is split over workgroups until they fill the CUs (mid_split); the parts (or
+// the one part) leave fp32 partial sums in the caller's workspace and
+// mid_reduce_kernel adds them in order, with the bias and the decode epilogue,
+// and puts right what an infinite x does to this kernel's sums.
 //
 // Bound by instruction issue, not bytes: of a step's 2250 cycles alone on a
 // CU, 830 are vector instructions (decoding 260, the outliers' addresses and
@@ -335,72 +335,131 @@ __global__ __launch_bounds__(64 * kMidWaves, 2) void qlinear_mid_kernel(QLArgs a
   }
 
   // C layout: lane l, element i -> row 16 gi + 4 (l / 16) + i, column l % 16
-  if (a.split > 1) {
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-      if (rbs[i] >= nrb) continue;
-      float* p = Ws[i]->part + (size_t)part * M * Ws[i]->N + rbs[i] * 16 + li;
-#pragma unroll
-      for (int gi = 0; gi < MG; gi++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const int m = 16 * gi + 4 * grp + e;
-          if (m < M) p[(size_t)m * Ws[i]->N] = acc[i][gi][e];
-        }
-    }
-    return;
-  }
-  float bv[2];
-#pragma unroll
-  for (int i = 0; i < 2; i++)
-    bv[i] = rbs[i] < nrb && Ws[i]->bias ? (float)bits_to_h(Ws[i]->bias[rbs[i] * 16 + li]) : 0.0f;
-  if (PAIR) {
-    if (rb0 >= nrb) return;
-#pragma unroll
-    for (int gi = 0; gi < MG; gi++)
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const int m = 16 * gi + 4 * grp + e;
-        const float g = (float)rn_h(acc[0][gi][e] + bv[0]), up = (float)rn_h(acc[1][gi][e] + bv[1]);
-        if (m < M) W.y[(size_t)m * W.N + rb0 * 16 + li] = h_to_bits(silu_mul_h(g, up));
-      }
-    return;
-  }
 #pragma unroll
   for (int i = 0; i < 2; i++) {
     if (rbs[i] >= nrb) continue;
-    const int n = rbs[i] * 16 + li;
+    float* p = Ws[i]->part + (size_t)part * M * Ws[i]->N + rbs[i] * 16 + li;
 #pragma unroll
     for (int gi = 0; gi < MG; gi++)
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         const int m = 16 * gi + 4 * grp + e;
-        if (m < M)
-          W.y[(size_t)m * W.N + n] = mid_epilogue(rn_h(acc[i][gi][e] + bv[i]), W.act,
-                                                  W.res ? W.res[(size_t)m * W.N + n] : (uint16_t)0, W.res != nullptr);
+        if (m < M) p[(size_t)m * Ws[i]->N] = acc[i][gi][e];
       }
   }
 }
 
-// The split parts' sums in order, the bias, one rounding, the epilogue: 4
-// columns a thread; grid row y is matrix y (the pair's gate).
-template <int PAIR>
+// The dequantized weight at (n, k): an outlier's value where the code is 0 and
+// the row's list has the column.
+template <int FMT>
+__device__ __forceinline__ float weight_at(const QLMat& w, int K, int n, int k) {
+  const uint32_t code = w.codes[tiled_offset(n, k, K >> 7)];
+  if (code == 0) {
+    int lo = w.row_ptr[n], hi = w.row_ptr[n + 1];
+    const int end = hi;
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (w.cols[mid] < k)
+        lo = mid + 1;
+      else
+        hi = mid;
+    }
+    if (lo < end && w.cols[lo] == k) return (float)bits_to_h(w.vals[lo]);
+  }
+  return (float)deq8<FMT>(code, 0u, scale2(w.scales[scale_index(w, n, k)]))[0];
+}
+
+__device__ __forceinline__ bool not_finite(uint32_t h) { return (h & 0x7C00u) == 0x7C00u; }
+
+// qlinear_mid_kernel multiplies x by zeros that stand for other values: an
+// outlier's decoded zero, the zeros beside an outlier's value in its B operand.
+// Where x is infinite they make NaN of sums that F.linear on the dequantized
+// weight leaves infinite (and the GEMM, which has each outlier's value in its
+// place).  A wave takes such sums v[c] of row m, columns n + c, again: a sum
+// with an infinite x is what its non-finite terms add up to, whatever the rest.
+// (Weights that are not finite themselves: all terms.)  Rows of x with a NaN,
+// or that are finite, keep theirs.  Every lane of the wave calls it.
+template <int FMT>
+__device__ __forceinline__ void mid_infinite(const QLArgs& a, const QLMat& w, int m, int n, bool live, float (&v)[4]) {
+  const int lane = threadIdx.x & 63, K = a.K;
+  const bool nan = live && (v[0] != v[0] || v[1] != v[1] || v[2] != v[2] || v[3] != v[3]);
+  uint64_t todo = __ballot(nan);
+  while (todo) {
+    const int mr = __builtin_amdgcn_readlane(m, __builtin_ctzll(todo));
+    const bool mine = nan && m == mr;
+    todo &= ~__ballot(mine);
+    bool odd = false;
+    if (mine) {
+      for (int b = 0; b < 4 * w.kg; b++) odd = odd || not_finite(w.scales[(size_t)n * w.kg + b]);
+      for (int p = w.row_ptr[n]; p < w.row_ptr[n + 4]; p++) odd = odd || not_finite(w.vals[p]);
+    }
+    const bool all = __ballot(odd) != 0;
+    float t[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    bool again = all, stop = false;
+    for (int k0 = 0; k0 < K && !stop; k0 += 512) {
+      const int k = k0 + 8 * lane;
+      u32x4 xv = (u32x4){0, 0, 0, 0};
+      if (k < K) xv = *reinterpret_cast<const u32x4*>(a.x + (size_t)mr * K + k);
+      uint32_t take = 0, nans = 0;
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const uint32_t h = (xv[j >> 1] >> (16 * (j & 1))) & 0xFFFFu;
+        take |= not_finite(h) ? 1u << j : 0u;
+        nans |= not_finite(h) && (h & 0x3FFu) ? 1u : 0u;
+      }
+      again = again || __ballot(take != 0) != 0;
+      if (__ballot(nans != 0)) {
+        again = false;
+        break;
+      }
+      if (all) take = k < K ? 0xFFu : 0u;
+      for (uint64_t from = __ballot(take != 0); from; from &= from - 1) {
+        const int s = __builtin_ctzll(from);
+        for (uint32_t q = (uint32_t)__builtin_amdgcn_readlane((int)take, s); q; q &= q - 1) {
+          const int j = __builtin_ctz(q);
+          const uint32_t word = j < 2 ? xv[0] : j < 4 ? xv[1] : j < 6 ? xv[2] : xv[3];
+          const float xk =
+              (float)bits_to_h((uint16_t)((uint32_t)__builtin_amdgcn_readlane((int)word, s) >> (16 * (j & 1))));
+          if (mine)
+#pragma unroll
+            for (int c = 0; c < 4; c++) t[c] = fmaf(xk, weight_at<FMT>(w, K, n + c, k0 + 8 * s + j), t[c]);
+        }
+      }
+      // NaN whatever else comes
+      stop = !__ballot(mine && (t[0] == t[0] || t[1] == t[1] || t[2] == t[2] || t[3] == t[3]));
+    }
+    if (mine && again)
+#pragma unroll
+      for (int c = 0; c < 4; c++)
+        if (v[c] != v[c]) v[c] = t[c];
+  }
+}
+
+// The parts' sums in order, the bias, one rounding, the epilogue: 4 columns a
+// thread; grid row y is matrix y (the pair's gate).
+template <int FMT, int PAIR>
 __global__ __launch_bounds__(256) void mid_reduce_kernel(QLArgs a) {
   const QLMat W = pick(a, (int)blockIdx.y);
   const int N = W.N;
   const int64_t mn = (int64_t)a.M * N;
-  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
-  if (i >= mn) return;
-  const int n = (int)(i % N);  // N is a multiple of 16: the 4 columns are of one row
-  auto sum = [&](const QLMat& w, float* v) {
+  const int64_t i0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  const bool live = i0 < mn;
+  const int64_t i = live ? i0 : 0;
+  const int m = (int)(i / N), n = (int)(i - (int64_t)m * N);  // N is a multiple of 16: the 4 columns are of one row
+  auto sum = [&](const QLMat& w, float (&v)[4]) {
     float4v s = *reinterpret_cast<const float4v*>(w.part + i);
     for (int p = 1; p < a.split; p++) s += *reinterpret_cast<const float4v*>(w.part + (size_t)p * mn + i);
 #pragma unroll
-    for (int j = 0; j < 4; j++) v[j] = s[j] + (w.bias ? (float)bits_to_h(w.bias[n + j]) : 0.0f);
+    for (int j = 0; j < 4; j++) v[j] = s[j];
+    const bool nan = v[0] != v[0] || v[1] != v[1] || v[2] != v[2] || v[3] != v[3];
+    if (__builtin_expect(__ballot(live && nan) != 0, 0)) mid_infinite<FMT>(a, w, m, n, live, v);
+#pragma unroll
+    for (int j = 0; j < 4; j++) v[j] += w.bias ? (float)bits_to_h(w.bias[n + j]) : 0.0f;
   };
   float v[4], u[4];
   sum(W, v);
   if (PAIR) sum(a.mat[1], u);
+  if (!live) return;
   uint16_t o[4];
 #pragma unroll
   for (int j = 0; j < 4; j++)
@@ -437,6 +496,16 @@ hipError_t launch_mid(const QLArgs& a, int pc, int mg, bool pair, hipStream_t s)
          : pc == 2 ? launch_mid<FMT, 2>(a, mg, pair, s) : launch_mid<FMT, 0>(a, mg, pair, s);
 }
 
+template <int FMT>
+hipError_t launch_reduce(const QLArgs& a, int64_t nmax, bool pair, hipStream_t s) {
+  const dim3 grid((unsigned)aq::ceil_div((int64_t)a.M * nmax, 1024), (unsigned)(pair ? 1 : a.count));
+  if (pair)
+    hipLaunchKernelGGL((mid_reduce_kernel<FMT, 1>), grid, dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL((mid_reduce_kernel<FMT, 0>), grid, dim3(256), 0, s, a);
+  return hipGetLastError();
+}
+
 }  // namespace
 
 namespace aqk {
@@ -451,8 +520,8 @@ static int64_t mid_units(const int64_t* Ns, int64_t count, bool pair) {
 
 // One workgroup per CU, in parts of at least 4 chunks: down_proj [4096,
 // 14336] at M = 64, 32 units, takes 70 us in 2 parts, 42 in 4, 31 in 8 and
-// 34 in 16; gate+up [28672, 4096], 224 units, 54 unsplit, 47 in 2 parts and
-// 49 in 4.
+// 34 in 16; gate+up [28672, 4096], 224 units, 54 in one, 47 in 2 parts and 49
+// in 4.
 int mid_split(const int64_t* Ns, int64_t count, int64_t K) {
   const int64_t units = mid_units(Ns, count, false);  // a pair splits as its members alone do
   const int64_t want = aq::ceil_div(aq::cu_count(), units);
@@ -472,13 +541,9 @@ hipError_t launch_qlinear_mid(QLArgs a, int fmt, int pc, bool pair, hipStream_t 
   const int mg = (int)aq::ceil_div(a.M, 16);
   const hipError_t e = fmt == AQ_FMT_E4M3 ? launch_mid<AQ_FMT_E4M3>(a, pc, mg, pair, s)
                                           : launch_mid<AQ_FMT_INT8>(a, pc, mg, pair, s);
-  if (e != hipSuccess || a.split == 1) return e;
-  const dim3 grid((unsigned)aq::ceil_div((int64_t)a.M * nmax, 1024), (unsigned)(pair ? 1 : a.count));
-  if (pair)
-    hipLaunchKernelGGL(mid_reduce_kernel<1>, grid, dim3(256), 0, s, a);
-  else
-    hipLaunchKernelGGL(mid_reduce_kernel<0>, grid, dim3(256), 0, s, a);
-  return hipGetLastError();
+  if (e != hipSuccess) return e;
+  return fmt == AQ_FMT_E4M3 ? launch_reduce<AQ_FMT_E4M3>(a, nmax, pair, s)
+                            : launch_reduce<AQ_FMT_INT8>(a, nmax, pair, s);
 }
 
 }  // namespace aqk

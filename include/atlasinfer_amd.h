@@ -256,7 +256,10 @@ int aq_zscore(const void* x, int64_t n, float eps, void* z, void* stats, void* s
  * against the outlier values); the GEMM
  * writes each outlier's fp16 value over its decoded zero in the weight tile
  * it multiplies.  Either way the result is x times the dequantized weight
- * accumulated in fp32, plus the bias, rounded once to fp16.
+ * accumulated in fp32, plus the bias, rounded once to fp16.  An x that is not
+ * finite gives the infinities and NaN of that product from the GEMM and from
+ * the linear that splits K; the GEMVs give NaN where an infinite x meets an
+ * outlier's decoded zero (and, with the block lists, in the 15 rows beside it).
  * workspace: aq_qlinear_workspace_size(M, N, K) bytes, 16-byte aligned, or
  * NULL.  A nonzero size means the GEMM would split K (2, 4 or 8 ways, chosen
  * from a time estimate of the shape on the current device), or 33 to 64 rows
@@ -346,7 +349,8 @@ int aq_qlinear_decode(const void* x, int64_t M, int64_t K, int fmt, int64_t coun
  * aq_qlinear_decode with a workspace, as aq_qlinear_grouped's: with
  * aq_qlinear_decode_workspace_size(M, sum of Ns, K) bytes (0 for most calls),
  * calls of 33 to 64 rows with the block lists split K over workgroups and keep
- * the fp32 partial sums there (NULL, or less: a smaller split, or none).
+ * the fp32 partial sums there (less: a smaller split; NULL, or too little: the
+ * GEMV).
  */
 int64_t aq_qlinear_decode_workspace_size(int64_t M, int64_t N, int64_t K);
 int aq_qlinear_decode_ws(const void* x, int64_t M, int64_t K, int fmt, int64_t count, const int64_t* Ns,
