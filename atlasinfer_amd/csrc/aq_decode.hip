@@ -51,6 +51,17 @@ __device__ __forceinline__ float row_bcast(float x, int n) {
                                             : __builtin_amdgcn_mov_dpp(u, 0x15C, 0xF, 0xF, false));
 }
 
+// The sum over the lanes of equal index in the wave's aligned groups of KV
+// lanes (8 or 16), in all of them.
+template <int KV>
+__device__ __forceinline__ float row_groups_sum(float x) {
+  if (KV == 8) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, x);
+    x += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(u, 0x128, 0xF, 0xF, false));  // row_ror:8, lane i ^ 8
+  }
+  return xlane_level_sum_f32<6>(xlane_level_sum_f32<5>(x));
+}
+
 // x * f rounded to fp16 (fp16 tensor times a Python float); f = 1 is exact.
 __device__ __forceinline__ f16 scale_h(f16 x, float f) { return f == 1.0f ? x : rn_h((float)x * f); }
 
@@ -88,26 +99,29 @@ __device__ __forceinline__ f16 rope_h(f16 x, f16 partner, bool lo, uint16_t c, u
 }
 
 // Splitting of the cache among workgroups.  A cache of at most 16 chunks of
-// 64 positions may be one span per head, its steps dealt to nw = 4 (or
-// fewer) waves of one workgroup that merge their results in LDS (no
-// second kernel): taken when a wave's serial share is short -- at most 4
-// chunk-units of work, a chunk costing G D / 64 units (scores and value
-// sums of 64 positions per lane, about 1000 vector instructions at G = 4,
-// D = 128) -- or when B Hkv >= 256 workgroups keep every SIMD busy anyway.
-// (Measured: OPT-1.3b batch 1, 32 heads of D = 64, 3 chunks: one span
-// 1168 against 1119 tok/s; Mistral-7B batch 32, 256 heads x batch rows:
-// 8116 against 7531; Mistral-7B batch 1, 8 key/value heads of G = 4,
-// D = 128, 12 chunks: 398 against 439, so split.)  Otherwise the cache is
-// split into spans of nt chunks, up to 4 waves each, nt the smallest power of
-// two that leaves ns = ceil(L / (64 nt)) <= 64 spans per head and
-// B Hkv ns <= 1024 workgroups (or one span for the whole cache);
-// decode_combine_kernel merges the spans.  (8 sequences of 4000 positions, 8
-// key/value heads: 9 spans a head 33.0 us, 17 spans 36.8, 33 spans 41.6: a
-// workgroup's start and merge cost as much as 100 positions.)
+// 64 positions is one span per head, its steps dealt to nw = 4 (or fewer)
+// waves of one workgroup that merge their results in LDS (no second kernel),
+// when a wave's serial share is short -- at most 8 steps, and at most 8
+// chunk-units, a chunk costing G D / 64 units -- or when B Hkv >= 128
+// workgroups share the CUs.
+// (G = 4, D = 128, 30 positions of 3 chunks: one span 7.5 us, split and
+// merged 9.4; 16 sequences x 8 heads at 300 of 7 chunks 13.3 against 18.1;
+// one sequence at 700 of 13 chunks 18.5 against 11.5, and 16 heads of G = 1,
+// 13 steps a wave, 9.9 against 8.1, so split.)  Otherwise
+// the cache is split into spans of nt chunks, up to 4 waves each, nt the
+// smallest power of two that leaves ns = ceil(L / (64 nt)) <= 64 spans per
+// head and B Hkv ns <= 384 workgroups (or one span for the whole cache);
+// decode_combine_kernel merges the spans.  A workgroup's start and merge cost
+// as much as 100 positions: 4 sequences x 8 heads at 1500 of 26 chunks 15.9 us
+// in 7 spans a head, 16.7 in 13, 19.8 in 26; 8 sequences x 8 heads at 4000
+// 30.0 in 5 spans, 31.7 in 9.
+// For the same reason spans of D = 64 that hold a whole short cache take one
+// wave instead of four once the workgroups fill the CUs without (2048 heads
+// at 130 positions 15.1 against 19.9 us, at 700 both 63.8).
 constexpr int kChunk = 64;
 constexpr int kOneSpanChunks = 16;
 constexpr int kMaxWaves = 4;  // one per SIMD: 8 would halve the registers a wave may hold (D = 128 then spills)
-constexpr int64_t kMaxGroups = 1024;
+constexpr int64_t kMaxGroups = 384;
 constexpr int64_t kMaxSpans = 64;
 
 struct Split {
@@ -123,7 +137,8 @@ inline Split split_of(int64_t B, int64_t Hkv, int64_t G, int64_t D, int64_t L) {
   const int64_t step = 4 * 64 / (D / 8);  // positions a wave takes at a time
   const int64_t nw1 = std::min<int64_t>(kMaxWaves, chunks * kChunk / step);
   const int64_t serial_units = (chunks + nw1 - 1) / nw1 * G * D / 64;
-  if (chunks <= kOneSpanChunks && (serial_units <= 4 || B * Hkv >= 256)) {
+  const int64_t serial_steps = (chunks * kChunk / step + nw1 - 1) / nw1;
+  if (chunks <= kOneSpanChunks && ((serial_units <= 8 && serial_steps <= 8) || B * Hkv >= 128)) {
     sp.nt = chunks;
     sp.ns = 1;
     sp.nw = nw1;
@@ -134,13 +149,16 @@ inline Split split_of(int64_t B, int64_t Hkv, int64_t G, int64_t D, int64_t L) {
     sp.ns = spans(sp.nt);
     sp.nw = std::min<int64_t>(kMaxWaves, sp.nt * kChunk / step);
   }
+  if (D == 64 && sp.ns == 1 && (B * Hkv >= 1024 || (B * Hkv >= 512 && chunks <= 5))) sp.nw = 1;
   sp.bytes = B * Hkv * sp.ns * sp.part_floats * 4;
   return sp;
 }
 
-// LDS of one workgroup of nw waves: per wave a chunk's softmax numerators
-// [G][64] and its merged result [G D + 2 G] (floats).
-inline size_t attention_lds(int64_t G, int64_t D, int64_t nw) { return (size_t)nw * (G * kChunk + G * D + 2 * G) * 4; }
+// LDS of one workgroup of nw waves, in floats: per wave the softmax numerators
+// of a step (D = 64: [G][32]; D = 128 passes them between lanes) and its merged
+// result [G D + 2 G].
+__host__ __device__ constexpr int numerators(int G, int D) { return D == 64 ? G * 32 : 0; }
+inline size_t attention_lds(int G, int D, int64_t nw) { return (size_t)nw * (numerators(G, D) + G * D + 2 * G) * 4; }
 
 // Workgroup (j, b, z) takes key/value head j of batch row b (query heads
 // j G .. j G + G - 1) and cache positions z span .. z span + span - 1
@@ -164,14 +182,12 @@ inline size_t attention_lds(int64_t G, int64_t D, int64_t nw) { return (size_t)n
 //           (reduce4): lane ln holds the score of row rs + RPW n_of(ch);
 //   values  weighted by their rows' numerators, broadcast to the row's lanes;
 //   sums    each lane keeps its share of the denominator.
-// Bound by HBM for long caches, by its chain of loads for short ones.  8
-// sequences of 4000 positions (8 key/value heads of 4 queries, 131 MB):
-// 32.6 us and 4.8 for the merge; 64 positions a step, a key row per lane and
-// no loads ahead took 34.1 and 9.1.  One sequence of 700: 9.0 us, 10.7 with
-// one wave per 64 positions.
+// Bound by HBM for long caches, by its chain of loads for short ones.  With
+// the merge of the spans, 8 sequences of 4000 positions (8 key/value heads of
+// 4 queries, 131 MB) take 30.0 us and one of 700 11.5; a wave per 64 positions,
+// a key row per lane and no loads ahead took 39.8 and 13.3.
 // Position pos's key and value come from k_new / v_new (the cache's copy is
-// this kernel's own store); positions past pos read k_new / v_new and weigh
-// zero.  Before use the queries are multiplied by q_scale (rounded to fp16;
+// this kernel's own store); positions past pos read as zero and weigh zero.  Before use the queries are multiplied by q_scale (rounded to fp16;
 // skipped for 1) and, given rcos / rsin (fp16 [L, D] tables), the queries
 // and the new key are rotated at position pos in the rotate-half form:
 // x' = fp16(fp16(x c) + fp16(r s)), r = (-x[D/2:], x[:D/2]) -- the order
@@ -185,8 +201,10 @@ inline size_t attention_lds(int64_t G, int64_t D, int64_t nw) { return (size_t)n
 // merge inside this kernel by the last span to arrive would need an
 // agent-scope release per span, which writes back the whole L2 of the
 // span's XCD; the kernel boundary orders the slots for free.)
+// (Registers: up to 128, four waves a SIMD, for G <= 2; one more and 1024
+// workgroups, G = 2, D = 64, come in two rounds.)
 template <int D, int G>
-__global__ __launch_bounds__(64 * kMaxWaves) void decode_attention_kernel(
+__global__ __launch_bounds__(64 * kMaxWaves, G <= 2 ? 4 : 2) void decode_attention_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_new, const uint16_t* __restrict__ v_new,
     uint16_t* __restrict__ k_cache, uint16_t* __restrict__ v_cache, const int64_t* __restrict__ pos_p, int H, int Hkv,
     int L, float scale, float q_scale, const uint16_t* __restrict__ rcos, const uint16_t* __restrict__ rsin, int nt,
@@ -196,6 +214,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void decode_attention_kernel(
   constexpr int NS = 4;         // loads of keys, and of values, a step
   constexpr int PS = RPW * NS;  // positions a step
   constexpr int PF = G * D + 2 * G;
+  static_assert(KV == 16 || numerators(G, D) == G * PS, "a step's numerators");
   const int j = blockIdx.x, b = blockIdx.y, z = blockIdx.z, t = threadIdx.x;
   const int nw = blockDim.x >> 6, ln = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -239,8 +258,8 @@ __global__ __launch_bounds__(64 * kMaxWaves) void decode_attention_kernel(
   __shared__ uint4 qs[G][KV];    // the group's queries, fp16
   __shared__ uint4 krot[KV];     // position pos's key as cached (last span only)
   extern __shared__ float dyn[];
-  float* w = dyn + wave * G * kChunk;     // this wave's numerators [G][PS] (D = 64)
-  float* res = dyn + nw * G * kChunk;     // the waves' results [nw][PF]
+  float* w = dyn + wave * numerators(G, D);  // this wave's numerators [G][PS] (D = 64)
+  float* res = dyn + nw * numerators(G, D);  // the waves' results [nw][PF]
 
   const uint16_t* cs = rcos ? rcos + pos * D : nullptr;
   const uint16_t* sn = rsin ? rsin + pos * D : nullptr;
@@ -354,43 +373,45 @@ __global__ __launch_bounds__(64 * kMaxWaves) void decode_attention_kernel(
     t0 += 2 * hop;
   }
 
-  // the wave's sums: the row groups' maxima meet, then the lanes' denominators
-  // and the RPW row groups' outputs
+  // waves whose first step lies past pos have nothing to add
+  const int na = (int)min((int64_t)nw, (pos - z0) / PS + 1);
+  if (wave < na) {
+    // the wave's sums: the row groups' maxima meet, then the lanes' denominators
+    // and the RPW row groups' outputs
 #pragma unroll
-  for (int g = 0; g < G; g++) {
-    const float mw = wave_group_max_f32<64>(m[g]);
-    const float c = m[g] == -INFINITY ? 0.0f : __expf(m[g] - mw);
-    m[g] = mw;
-    lt[g] *= c;
+    for (int g = 0; g < G; g++) {
+      const float mw = wave_group_max_f32<64>(m[g]);
+      const float c = m[g] == -INFINITY ? 0.0f : __expf(m[g] - mw);
+      m[g] = mw;
+      lt[g] *= c;
 #pragma unroll
-    for (int h = 0; h < 8; h++) acc[g][h] *= c;
-    lt[g] = wave_group_sum_f32<64>(lt[g]);
+      for (int h = 0; h < 8; h++) acc[g][h] *= c;
+      lt[g] = wave_group_sum_f32<64>(lt[g]);
 #pragma unroll
-    for (int h = 0; h < 8; h++)
+      for (int h = 0; h < 8; h++) acc[g][h] = row_groups_sum<KV>(acc[g][h]);
+    }
+    if (nw == 1 && nact == 1) {
+      if (rs == 0) {
 #pragma unroll
-      for (int off = KV; off < 64; off <<= 1) acc[g][h] += __shfl_xor(acc[g][h], off);
-  }
-  if (nw == 1 && nact == 1) {
+        for (int g = 0; g < G; g++)
+#pragma unroll
+          for (int h = 0; h < 8; h++) o[g * D + 8 * ch + h] = h_to_bits(rn_h(acc[g][h] / lt[g]));
+      }
+      return;
+    }
+    float* pp = nw == 1 ? part + (kv * ns + z) * PF : res + wave * PF;
     if (rs == 0) {
 #pragma unroll
       for (int g = 0; g < G; g++)
 #pragma unroll
-        for (int h = 0; h < 8; h++) o[g * D + 8 * ch + h] = h_to_bits(rn_h(acc[g][h] / lt[g]));
+        for (int h = 0; h < 8; h++) pp[g * D + 8 * ch + h] = acc[g][h];
     }
-    return;
-  }
-  float* pp = nw == 1 ? part + (kv * ns + z) * PF : res + wave * PF;
-  if (rs == 0) {
+    if (ln == 0) {
 #pragma unroll
-    for (int g = 0; g < G; g++)
-#pragma unroll
-      for (int h = 0; h < 8; h++) pp[g * D + 8 * ch + h] = acc[g][h];
-  }
-  if (ln == 0) {
-#pragma unroll
-    for (int g = 0; g < G; g++) {
-      pp[G * D + g] = m[g];
-      pp[G * D + G + g] = lt[g];
+      for (int g = 0; g < G; g++) {
+        pp[G * D + g] = m[g];
+        pp[G * D + G + g] = lt[g];
+      }
     }
   }
   if (nw == 1) return;  // the span's partial is in part; decode_combine_kernel merges
@@ -401,9 +422,9 @@ __global__ __launch_bounds__(64 * kMaxWaves) void decode_attention_kernel(
   for (int i = t; i < G * D + G; i += 64 * nw) {
     const int g = i < G * D ? i / D : i - G * D;
     float mx = -INFINITY;
-    for (int v = 0; v < nw; v++) mx = fmaxf(mx, res[v * PF + G * D + g]);
+    for (int v = 0; v < na; v++) mx = fmaxf(mx, res[v * PF + G * D + g]);
     float num = 0.0f, den = 0.0f;
-    for (int v = 0; v < nw; v++) {
+    for (int v = 0; v < na; v++) {
       const float mv = res[v * PF + G * D + g];
       const float f = mv == -INFINITY ? 0.0f : __expf(mv - mx);
       den = fmaf(res[v * PF + G * D + G + g], f, den);

@@ -64,6 +64,25 @@ def test_long_caches(B, Hkv, G, D, L, pos):
     _run(B, Hkv, G, D, L, pos, pos)
 
 
+# both sides of the splitting rule's lines, with positions that leave waves
+# without a step, or with the position alone
+@pytest.mark.parametrize("B,Hkv,G,D,L,poss", [
+    (64, 16, 1, 64, 320, (0, 31, 32, 130, 319)),     # 1024 heads: one wave
+    (64, 16, 2, 64, 832, (5, 700)),
+    (32, 16, 2, 64, 320, (33, 319)),                 # 512 heads, 5 chunks: one wave
+    (32, 16, 1, 64, 321, (40, 320)),                 # 6 chunks: four
+    (16, 8, 4, 128, 448, (0, 15, 16, 47, 48, 300)),  # 128 heads: one span of four waves
+    (127, 1, 4, 128, 448, (16, 300)),                # 127: split
+    (1, 4, 8, 64, 192, (31, 32, 190)),               # 8 chunk-units a wave: one span
+    (1, 16, 1, 128, 832, (700,)),                    # 13 steps a wave: split
+    (25, 8, 1, 64, 4160, (64, 4100)),                # 200 heads: a span longer than the cache
+    (8, 8, 4, 128, 1664, (511, 512, 1500)),          # spans of 8 chunks
+])
+def test_splitting(B, Hkv, G, D, L, poss):
+    for pos in poss:
+        _run(B, Hkv, G, D, L, pos, pos)
+
+
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("pos,low", [(40, 32), (700, 650), (4000, 64)])
 def test_scores_of_minus_infinity(D, pos, low):
