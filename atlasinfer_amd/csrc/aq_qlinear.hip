@@ -26,6 +26,9 @@
 //    LDS (details at its kernel below), since x is then comparable to or
 //    larger than the codes it multiplies.  (M = 1..5 re-read
 //    x per tile row above; decode stages it in LDS once per workgroup.)
+//  * 33 <= M <= 64, given the outlier block lists, on the grids mid_takes names:
+//    the linear split over K (aq_qlinear_mid.hip).  Other short grids with the
+//    lists, decode steps aside, take the GEMM.
 //  * M > 64: dequant-GEMM (details at its kernel below): 128 or 256 rows of
 //    x by 128 output columns per workgroup, x and decoded weights staged in
 //    LDS in MFMA operand order, each outlier written over its decoded zero,
@@ -67,15 +70,14 @@ __device__ __forceinline__ GemvIn gemv_in(const QLArgs& a, int off = 0) {
 }
 
 constexpr int kGemvMaxM = 64;   // larger M takes the GEMM
-// From 33 rows of x on, grids of fewer than 384 tile rows take the GEMM when the
-// caller passes the outlier block lists: the GEMV's x stages for 64 rows fit
-// LDS only with 4 waves per tile row, which leaves half the CUs idle there
-// (down_proj [4096, 14336] at M = 33..64: 78 us against 29 with the GEMM;
-// q/o and k/v about equal; taller grids such as grouped q/k/v or gate+up stay
-// faster on the GEMV)
+// From 33 rows of x on, grids of fewer than 384 tile rows take the GEMM, or the
+// linear split over K (mid_takes), when the caller passes the outlier block
+// lists: the GEMV's x stages for 64 rows fit LDS only with 4 waves per tile row,
+// which leaves half the CUs idle there (down_proj [4096, 14336] at M = 64: 88 us
+// against 34 with the GEMM and 29 split; taller grids such as grouped q/k/v or
+// gate+up stay faster on the GEMV than on the GEMM)
 constexpr int kGemvShortMaxM = 32;
 constexpr int kGemvShortRows = 384;
-constexpr int kGemvTallRows = 768;
 constexpr int kGemvXMinM = 6;   // from here on the GEMV shares x through LDS (qlinear_gemv_x_kernel)
 constexpr int kGemvUnroll = 2;  // 128-wide K chunks per wave with loads in flight together
 constexpr int kGemvDirectMaxM = kGemvXMinM - 1;  // rows of x qlinear_gemv_kernel takes
@@ -1964,26 +1966,37 @@ hipError_t launch_gemm_wide(const QLArgs& a, int fmt, bool per_channel, bool den
 
 // Whether 33 to 64 rows of x on a grid of `blocks` tile rows go to the linear
 // split over K (aq_qlinear_mid.hip), given the block lists and a workspace.
-// Short grids (below 384 tile rows) do: at M = 64 in a decode step o_proj
-// 25 -> 18.4 us and down_proj 90 -> 31 against the shared-x GEMV; against the
-// GEMM, which plain calls took, on up to 256 tile rows [4096, 14336] 33.5 ->
-// 27.9 at M = 33 and 33.2 -> 31.1 at 64, in blocks of 128 36.3 -> 27.6 and
-// 36.6 -> 31.9, [2048, 8192] 22.4 -> 18.3 and 23.0 -> 21.0, [4096, 4096]
-// 16.5 -> 15.9 and 18.5 -> 18.3 ([6000, 4096], 375 tile rows, 23.4 -> 25.9:
-// the GEMM's).  Plain calls of 49 rows or more with K below 4096 stay with it
-// ([2048, 2048] at M = 64 14.4 against 15.1), and weights of heavy tails
-// (1.4 % outliers, up to 35 in a block: [4096, 14336] at M = 64 35.1 against
-// 53.6; the shared-x GEMV, which decode steps had, 84).  Decode steps also
-// take it on tall grids (gate+up
-// 54.5 -> 47 at M = 64; a plain call there has no workspace, and unsplit it
-// gains nothing); between the two the shared-x GEMV stays ahead (q/k/v 22.3
-// against 24.5, [8192, 2048] 14.6 against 19).  Two bands of up to 64 rows did
-// not carry it past 64: [8192, 2048] at M = 128 24.7 us against the GEMM's
-// 22.7, [4096, 14336] 44.9 against 36.2.
+//
+// Plain calls, which have the GEMM on short grids (below 384 tile rows), do on
+// up to 256 tile rows: [4096, 14336] 34.2 -> 26.9 us at M = 33 and 33.9 -> 28.7
+// at 64, [2048, 8192] 22.7 -> 18.9 and 23.5 -> 21.9, [4096, 4096] 16.8 -> 15.5
+// and 19.4 -> 18.0 ([6000, 4096], 375 tile rows, 23.4 -> 25.9: the GEMM's).
+// Those of 49 rows or more with K below 4096 stay with the GEMM ([2048, 2048]
+// at M = 64 14.4 against 15.1), and weights of heavy tails (1.4 % outliers, up
+// to 35 in a block: [4096, 14336] at M = 64 35.1 against 53.6).  Two bands of
+// up to 64 rows did not carry it past 64: [8192, 2048] at M = 128 24.7 us
+// against the GEMM's 22.7, [4096, 14336] 44.9 against 36.2.
+//
+// Decode steps, which have the shared-x GEMV, do on up to 256 tile rows with K
+// from 4096 on (2560 from 49 rows on), on more below 384 from 12288 on:
+// [4096, 14336] at M = 33 / 64 47.1 -> 26.8 / 58.3 -> 30.1 us, [4096, 4096]
+// 17.2 -> 15.5 / 21.6 -> 18.2, [1024, 2560] at 49 16.8 -> 12.5, [5120, 13824]
+// 46.7 -> 34.5 / 58.0 -> 38.4; not [2048, 2048] at 33 11.7 -> 12.6, [5120, 1024]
+// 8.6 -> 12.0, [6000, 4096] 17.5 -> 20.0, [5120, 5120] 21.8 -> 22.7.  Heavy
+// tails (up to 40 outliers in a block) move with them there ([4096, 14336]
+// 72.4 -> 54.0 / 88.5 -> 59.0, [4096, 4096] 24.5 -> 23.6 / 30.3 -> 26.7, in
+// blocks of 64 25.8 -> 26.6 / 32.4 -> 32.1), so the count, which these calls
+// don't have, would not change the choice.  And from 49 rows on on tall grids
+// that leave few CUs empty: gate+up [28672, 4096] at M = 64 53.4 -> 42.4,
+// [24576, 2048] 33.4 -> 32.4, [32768, 2048] 33.2 -> 31.1, with heavy tails 202 ->
+// 82 (up to 48 rows 37.9 -> 39.4, in blocks of 128 40.8 -> 45.1; [14336, 4096],
+// 896 tile rows, 29.1 -> 33.0; [24576, 1024] 20.9 -> 22.8).
 bool mid_takes(int64_t M, int64_t blocks, int64_t K, bool decode) {
   if (M < kMidMinM || M > kMidMaxM) return false;
-  if (decode) return blocks < kGemvShortRows || blocks >= kGemvTallRows;
-  return blocks <= kMidPlainMaxRows && (M <= kMidPlainMaxM || K >= kMidPlainMinK);
+  const bool low = M <= 48;
+  if (!decode) return blocks <= kMidMaxRows && (low || K >= 4096);
+  if (blocks >= kGemvShortRows) return blocks >= kMidTallRows && !low && K >= 2048;
+  return K >= (blocks > kMidMaxRows ? 12288 : low ? 4096 : 2560);
 }
 
 }  // namespace
@@ -2076,9 +2089,10 @@ static int qlinear_grouped_impl(const void* x, int64_t M, int64_t K, int fmt, in
   for (int i = (int)count; i <= kMaxGroup; i++) a.first[i] = (int)blocks;
   a.split = 1;
   if (fz) {
-    // decode: the M = 1 GEMV with x in LDS (every prologue) or the shared-x
-    // GEMV for 6 <= M <= 64 (epilogue only: each of its workgroups stages all
-    // of x, so a prologue there would be computed once per workgroup)
+    // decode: the M = 1 GEMV with x in LDS (every prologue) or, for 6 <= M <=
+    // 64, the shared-x GEMV or the linear split over K (epilogue only: each of
+    // the GEMV's workgroups stages all of x, so a prologue there would be
+    // computed once per workgroup)
     AQ_CHECK_ARG((M == 1 && K <= kGemvX1MaxK) || (M >= kGemvXMinM && M <= kGemvMaxM),
                  "aq_qlinear_decode: M = 1 with K <= %d, or 6 <= M <= 64 (M=%lld K=%lld)", kGemvX1MaxK, (long long)M,
                  (long long)K);
@@ -2120,7 +2134,7 @@ static int qlinear_grouped_impl(const void* x, int64_t M, int64_t K, int fmt, in
   const bool gemv = M <= kGemvShortMaxM || (M <= kGemvMaxM && (blocks >= kGemvShortRows || !have_lists));
   bool mid = mid_takes(M, blocks, K, fz != nullptr) && tile_ptrs && tile_ents;
   // more outliers than that in a block take rounds of their own, in which
-  // nothing is in flight; decode calls don't know the count
+  // nothing is in flight (the GEMM has none; the decode steps' GEMV has, see mid_takes)
   for (int i = 0; i < count && mid && !fz; i++) mid = tile_maxes && tile_maxes[i] <= kMidPlainMaxOutl;
   if (mid) {
     const bool pair = a.mat[0].act == 2;
@@ -2134,7 +2148,7 @@ static int qlinear_grouped_impl(const void* x, int64_t M, int64_t K, int fmt, in
     int split = workspace && (uintptr_t)workspace % 16 == 0 ? want : 0;
     while (split > 0 && workspace_bytes < split * outs * 4) split--;
     // short grids pay only when split
-    if (lists && (split > 1 || (split == want && blocks >= kGemvTallRows))) {
+    if (lists && (split > 1 || (split == want && blocks >= kMidTallRows))) {
       a.split = split;
       float* p = (float*)workspace;
       for (int i = 0; i < count; i++) {
@@ -2237,7 +2251,7 @@ extern "C" int aq_qlinear_decode_ws(const void* x, int64_t M, int64_t K, int fmt
                                     float eps, const void* const* residuals, const int32_t* relu, void* workspace,
                                     int64_t workspace_bytes, void* stream) {
   const DecodeFuse fz{prologue, x2, norm_weight, norm_bias, eps, residuals, relu};
-  // no tile_max: the decode GEMVs never take the GEMM
+  // no tile_max: decode calls never take the GEMM
   return qlinear_grouped_impl(x, M, K, fmt, count, Ns, codes, scales, Gs, row_ptrs, cols, vals, tile_ptrs, tile_ents,
                               nullptr, biases, ys, workspace, workspace_bytes, stream, &fz);
 }

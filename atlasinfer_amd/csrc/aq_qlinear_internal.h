@@ -137,9 +137,9 @@ constexpr int kBufferDword3 = 0x00020000;      // raw (untyped) buffer access on
 // parts of K (partial sums at a.mat[i].part, also of one part); pc: the
 // scale mode of the GEMVs.  mid_split: the parts a launch wants.
 constexpr int kMidMinM = 33, kMidMaxM = 64;
-// plain calls: up to so many tile rows and outliers in a 16 x 64 block, and so
-// many rows of x or from such a K on
-constexpr int kMidPlainMaxRows = 256, kMidPlainMaxOutl = 20, kMidPlainMaxM = 48, kMidPlainMinK = 4096;
+// its short grids' and its tall grids' tile rows (192 units of 128 columns), and
+// the most outliers in a 16 x 64 block of a plain call
+constexpr int kMidMaxRows = 256, kMidTallRows = 1536, kMidPlainMaxOutl = 20;
 int mid_split(const int64_t* Ns, int64_t count, int64_t K);
 hipError_t launch_qlinear_mid(QLArgs a, int fmt, int pc, bool pair, hipStream_t s);
 

@@ -95,6 +95,18 @@ def test_bad_arguments_return_einval_with_message(lib):
     assert lib.aq_tile_codes(p, 20, 128, p, None) == AQ_EINVAL
 
 
+def test_decode_workspace_rule(lib):
+    """The sizes say which decode calls split K: 33 to 64 rows, long rows on
+    short grids, and from 49 rows on tall grids."""
+    size = lib.aq_qlinear_decode_workspace_size
+    for M, N, K, takes in [(32, 4096, 4096, 0), (33, 4096, 4096, 1), (64, 4096, 14336, 1), (65, 4096, 4096, 0),
+                           (48, 4096, 3968, 0), (49, 4096, 2560, 1), (49, 4096, 2432, 0), (64, 4112, 4096, 0),
+                           (33, 6128, 12288, 1), (64, 6144, 14336, 0), (64, 14336, 4096, 0), (48, 28672, 4096, 0),
+                           (49, 24576, 2048, 1), (49, 24560, 2048, 0), (64, 24576, 1920, 0), (64, 4096, 4100, 0)]:
+        b = size(M, N, K)
+        assert (b > 0) == bool(takes) and b % (M * N * 4) == 0, (M, N, K, b)
+
+
 def test_workspace_sizes(lib):
     assert lib.aq_quantize_workspace_size(4096 * 4096, 4096) >= 4096 * 4096 * 6
     assert lib.aq_quantize_workspace_size(0, 128) == 0

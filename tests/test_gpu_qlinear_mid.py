@@ -1,7 +1,8 @@
-"""qlinear_decode at 33 to 64 rows, where short and tall grids split K over
-workgroups: against the float64 product of x and the dequantized weight, with
-every split the workspace allows (the parts' sums differ in order only), the
-decode epilogue, ragged last units, odd part lengths and crowded blocks."""
+"""qlinear_decode and plain linears at 33 to 64 rows, where some grids split K
+over workgroups (aq_qlinear_decode_workspace_size says which): against the
+float64 product of x and the dequantized weight, with every split the workspace
+allows (the parts' sums differ in order only), the decode epilogue, ragged last
+units, odd part lengths and crowded blocks."""
 import ctypes
 
 import numpy as np
@@ -46,7 +47,11 @@ def _close(y, x, deq, bias=None):
 # scales per row, per chunk and finer, both row-group counts
 @pytest.mark.parametrize("N,K,G,M,fmt", [(48, 896, -1, 33, "e4m3"), (272, 1408, 128, 48, "e4m3"),
                                          (4096, 2944, 64, 49, "e4m3"), (1024, 4096, 256, 64, "int8"),
-                                         (256, 9472, -1, 64, "e4m3"), (12304, 1024, -1, 40, "e4m3")])
+                                         (256, 9472, -1, 64, "e4m3"), (12304, 1024, -1, 40, "e4m3"),
+                                         # the decode rule's own side: 33, 35, 21, 96 and 17 chunks
+                                         (48, 4224, -1, 33, "e4m3"), (272, 4480, 128, 48, "e4m3"),
+                                         (4096, 2688, 64, 49, "e4m3"), (4112, 12288, -1, 40, "int8"),
+                                         (24592, 2176, 128, 64, "e4m3"), (32784, 2048, -1, 49, "e4m3")])
 def test_mid_matches_dequantized_product(N, K, G, M, fmt):
     q, deq = _weight(N, K, G, fmt, N + K)
     x = _x(M, K, M)
@@ -81,6 +86,50 @@ def test_mid_every_split():
         _close(y, x, deq)
 
 
+def _decode_ws(x, q, nbytes):
+    """aq_qlinear_decode_ws with a workspace of ``nbytes``."""
+    (M, K), N = x.shape, q.original_shape[0]
+    L, arr = _lib.load(), _lib.ptr_array
+    tp, te, _ = AQ.outlier_tiles(q, DEV)
+    codes = AQ.kernel_codes(q, DEV)
+    ws = torch.full((nbytes,), 0xFF, dtype=torch.uint8, device=DEV)  # NaN where nothing is written
+    y = torch.empty(M, N, dtype=torch.float16, device=DEV)
+    _lib.check(L.aq_qlinear_decode_ws(
+        x.data_ptr(), M, K, _lib.FORMATS[q.code_format], 1, arr([N], ctypes.c_int64), arr([codes.data_ptr()]),
+        arr([q.scale_factors.data_ptr()]), arr([q.block_size], ctypes.c_int64), arr([q.outlier_row_ptr.data_ptr()]),
+        arr([q.outlier_cols.data_ptr()]), arr([q.fp16_outliers.data_ptr()]), arr([tp.data_ptr()]),
+        arr([te.data_ptr()]), arr([None]), arr([y.data_ptr()]), 0, None, None, None, ctypes.c_float(0), None, None,
+        ws.data_ptr(), nbytes, _lib.stream_of(DEV)), "aq_qlinear_decode_ws")
+    return y
+
+
+# two parts of 62 to 66 and of 129 chunks: the registers that hold 64 chunks'
+# outlier ranges are filled again on the way, once and twice
+@pytest.mark.parametrize("M", [33, 64])
+@pytest.mark.parametrize("chunks,G,fmt", [(124, -1, "e4m3"), (126, 128, "int8"), (128, 64, "e4m3"), (130, -1, "e4m3"),
+                                          (132, 128, "e4m3"), (258, -1, "int8")])
+def test_mid_long_parts(chunks, G, fmt, M):
+    N, K = 144, 128 * chunks
+    q, deq = _weight(N, K, G, fmt, chunks)
+    x = _x(M, K, M)
+    _close(_decode_ws(x, q, 2 * M * N * 4), x, deq)
+
+
+@pytest.mark.parametrize("N,K,M", [(80, 4224, 33), (1616, 4096, 64), (12304, 2048, 50), (16400, 2048, 64)])
+def test_mid_pair_is_its_members(N, K, M):
+    """gate and up as a pair sum as they do alone: bit for bit aq_silu_mul of the two."""
+    (g, _), (u, _) = _weight(N, K, 128, "e4m3", 1), _weight(N, K, 128, "e4m3", 2)
+    x = _x(M, K, 2)
+    codes = [q.fp8_data.view(torch.uint8) for q in (g, u)]
+    assert int(_lib.load().aq_qlinear_decode_workspace_size(M, 2 * N, K)) > 0
+    a = AW.qlinear_decode(x, [g, u], [None, None], codes, swiglu_pair=True)[0]
+    yg, yu = AW.qlinear_decode(x, [g, u], [None, None], codes)
+    want = torch.empty_like(yg)
+    _lib.check(_lib.load().aq_silu_mul(yg.data_ptr(), yu.data_ptr(), want.data_ptr(), M * N, _lib.stream_of(DEV)),
+               "aq_silu_mul")
+    assert torch.equal(a, want)
+
+
 def test_mid_grouped_and_swiglu_pair():
     """Members of different sizes in one launch; gate and up as a pair, split and not."""
     K, M = 1664, 50
@@ -95,7 +144,9 @@ def test_mid_grouped_and_swiglu_pair():
         a = AW.qlinear_decode(x, [g, u], [None, None], codes, swiglu_pair=True)[0]
         yg, yu = AW.qlinear_decode(x, [g, u], [None, None], codes)
         want = torch.nn.functional.silu(yg.float()).half() * yu
-        assert (a.float() - want.float()).abs().max() <= 2.0 ** -9 * want.float().abs().max()
+        # silu rounded to fp16 one way or the other, then the product
+        ulp = np.spacing(np.abs(want.cpu().numpy()).astype(np.float16)).astype(np.float32)
+        assert (np.abs(a.float().cpu().numpy() - want.float().cpu().numpy()) <= 2 * ulp).all()
 
 
 def test_mid_crowded_blocks():
@@ -119,7 +170,7 @@ def test_mid_plain(N, K, G, fmt, M, thr):
     tiles = AQ.outlier_tiles(q, DEV)
     y = AW.qlinear(x, q, bias, codes=AQ.kernel_codes(q, DEV), tiles=tiles)
     _close(y, x, deq, bias)
-    if int(tiles[2]) <= 20 and (M <= 48 or K >= 4096):  # the decode call's sums
+    if int(tiles[2]) <= 20 and K >= 4096:  # the decode call's sums
         assert torch.equal(y, AW.qlinear_decode(x, [q], [bias], [AQ.kernel_codes(q, DEV)], tiles=[tiles])[0])
 
 
