@@ -21,10 +21,11 @@
 // mid_reduce_kernel adds them in order, with the bias and the decode epilogue,
 // and puts right what an infinite x does to this kernel's sums.
 //
-// Bound by instruction issue, not bytes: of a step's 2250 cycles alone on a
-// CU, 830 are vector instructions (decoding 260, the outliers' addresses and
-// selects about as many) and 450 MFMAs; without outliers [28672, 4096] at
-// M = 64 takes 37 us instead of 47, without x, outliers and MFMAs 27.
+// Bound by instruction issue, not bytes: gate+up [28672, 4096] at M = 64 takes
+// 39 us for 119 MB.  A wave's step is 259 vector instructions (1061 cycles;
+// decoding and the outliers' addresses and selects the most of them), 40 MFMAs
+// (644) and 32 LDS reads; a third of its time it waits to issue, a third for
+// memory or the barrier (profiles/qlinear_mid_llama3_8b_m64_counters.txt).
 #include <algorithm>
 
 #include "aq_common.h"

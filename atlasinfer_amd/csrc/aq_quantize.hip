@@ -247,9 +247,10 @@ __device__ float outlier_cut(f16 den, f16 thr) {
 // the step lies between c0 and c0 + 2, so four patterns from c0 - 1 on hold
 // it.  (Four from c0 - 2 on missed it for one block in twenty, and with 16
 // blocks of 128 to a wave every second wave bisected: with the sums' exact
-// cases below, 1096 -> 787 VALU instructions a wave and 63 -> 51 us for a
-// 14336 x 4096 weight.)  Subnormal thresholds
-// and products may fall outside: those bisect.
+// cases below and the outliers staged by wave, 1056 -> 667 VALU instructions a
+// wave and 65 -> 50 us for a 14336 x 4096 weight,
+// profiles/quantize_kernel_g128_llama3_8b_trace.txt.)  Subnormal thresholds and
+// products may fall outside: those bisect.
 template <int TAU>
 __device__ float outlier_cut_team(f16 den, f16 thr) {
   const float fden = (float)den;
@@ -1372,8 +1373,9 @@ Workspace carve(void* ws, int64_t padded) {
   return Workspace{(uint32_t*)ws, (int32_t*)((char*)ws + align256(padded * 4))};
 }
 
-// (2 bytes an element more than the stage takes: the size has been this much
-// for callers that compute with it)
+// 6 bytes an element, of which the stage takes 4: the size is part of the
+// entry points' behaviour (test_capi.py holds it to at least that), as when
+// columns and values were staged apart
 int64_t workspace_bytes(int64_t padded, int64_t nblocks) {
   return align256(padded * 4) + align256(padded * 2) + align256((aq::ceil_div(nblocks, kScanChunk) + 1) * 4);
 }

@@ -38,7 +38,7 @@ __device__ __forceinline__ int lower_bound_i32(const int32_t* a, int lo, int hi,
 // Raise *p to at least v.  Many workgroups raise one word: a relaxed read
 // first skips the atomic when the word is already that large (it only
 // grows, so skipping keeps the maximum), since atomics on one address are
-// serialized in memory at about 8 ns each.
+// serialized in memory at 8 to 9 ns each (see launch_tile_max).
 __device__ __forceinline__ void raise_to(int32_t* p, int v) {
   if (v > __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(p, v);
 }
@@ -183,9 +183,9 @@ __device__ __forceinline__ void tile_row_sort(const Src& src, int rb, int nch, i
 // each list's word from its finished tile_ptr (n blocks): a launch of its
 // own, a few workgroups a list, for launches of more than kRaiseTileRows tile
 // rows.  Raised by the sort's workgroups, which are all resident at once and
-// so all find the old value, the atomics on one word (8 ns each, in memory)
-// took longer than the sort: a layer's six weights, 2432 tile rows, 31.5 us
-// with them, 10.5 without, and this launch takes 3.8.  Fewer tile rows raise
+// so all find the old value, the atomics on one word took longer than the
+// sort: a layer's six weights, 2432 tile rows, 31.5 us with them, 10.5
+// without (8.6 ns each), and this launch takes 3.8.  Fewer tile rows raise
 // it themselves, which costs less than a launch.  Defined in aq_layout.hip.
 constexpr int kRaiseTileRows = 320;
 constexpr int kMaxTileMax = 8;

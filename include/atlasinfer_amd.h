@@ -150,7 +150,8 @@ int aq_outlier_tiles(const int32_t* row_ptr, const int32_t* cols, const void* va
 
 /*
  * aq_quantize_finish (with cols) and aq_outlier_tiles of the same weight in
- * one launch, read straight from the quantize workspace: the flat list and
+ * one pass, read straight from the quantize workspace (one launch; a second
+ * one for tile_max above 320 tile rows): the flat list and
  * the block lists, bit for bit those of the two calls.  For weights
  * quantized with blocks that tile the rows (K % G == 0) and whose [N, K]
  * view has N % 16 == 0 and K % 64 == 0 (every weight quantized into the
@@ -167,7 +168,7 @@ int aq_quantize_finish_tiles(int64_t numel, int64_t G, int64_t K, const int32_t*
 
 /*
  * aq_quantize_finish_tiles for up to 8 weights of one block size G and row
- * length K in one launch (the members of an aq_quantize_grouped call): per
+ * length K in one pass (the members of an aq_quantize_grouped call): per
  * member i the arguments of aq_quantize_finish_tiles (numels[i],
  * block_offs[i], nnzs[i], workspaces[i] of ws_bytes[i], flat_idx[i],
  * vals[i], cols[i], tile_ptrs[i], tile_ents[i]); tile_max, if not NULL,
@@ -247,13 +248,15 @@ int aq_zscore(const void* x, int64_t n, float eps, void* z, void* stats, void* s
  *   M <= 5        dequant-GEMV, each 16-row tile row reading x directly;
  *   6 <= M <= 64  dequant-GEMV sharing x through LDS, except that from
  *                 M = 33 on, grids of fewer than 384 tile rows (N < 6144,
- *                 summed over a group) take the dequant-GEMM when tile_ptr
- *                 and tile_ent are given;
+ *                 summed over a group) take, when tile_ptr and tile_ent are
+ *                 given, the linear split over K (up to 256 tile rows, at most
+ *                 48 rows of x or K >= 4096, tile_max <= 20, and a workspace
+ *                 for two parts or more) or else the dequant-GEMM;
  *   M > 64        dequant-GEMM (tile_ptr, tile_ent required).
  * The GEMVs add the outliers from the CSR lists in fp32, except the shared-x
  * GEMV given the block lists (M <= 32, or groups under 768 tile rows), which
  * multiplies each chunk's outliers with one more MFMA (x columns gathered
- * against the outlier values); the GEMM
+ * against the outlier values), as the linear split over K does; the GEMM
  * writes each outlier's fp16 value over its decoded zero in the weight tile
  * it multiplies.  Either way the result is x times the dequantized weight
  * accumulated in fp32, plus the bias, rounded once to fp16.  An x that is not
@@ -298,7 +301,7 @@ int aq_qlinear_grouped(const void* x, int64_t M, int64_t K, int fmt, int64_t cou
  * device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  No counterpart in the reference.
  * Same arguments, kernels and results as aq_qlinear given a workspace of
- * AQ_NOALLOC_SCRATCH_BYTES: the GEMM's split-K partial sums go to a static
+ * AQ_NOALLOC_SCRATCH_BYTES: the partial sums of a split over K go to a static
  * device array of that size inside the library, one per GPU, held from the
  * first use on a GPU until the process ends.  The split is planned within
  * that size (as aq_qlinear's within its workspace), so no call is too large
@@ -315,9 +318,10 @@ int aq_qlinear_noalloc(const void* x, int64_t M, int64_t K, int64_t N, const voi
 /*
  * One decode-step launch of up to 4 quantized linears sharing x (M rows:
  * 1 with K <= 16384, or 6 <= M <= 64), with the layer's neighbouring
- * elementwise work folded in: the GEMV paths of aq_qlinear_grouped (the
- * reference's QuantizedLinear.forward, integration/atlas_wrappers.py:56-67,
- * at decode sizes) plus
+ * elementwise work folded in: the GEMV paths of aq_qlinear_grouped, or with
+ * aq_qlinear_decode_ws the linear split over K (the reference's
+ * QuantizedLinear.forward, integration/atlas_wrappers.py:56-67, at decode
+ * sizes), plus
  *   prologue  what the linears read instead of x:
  *             0  x as given
  *             1  RMSNorm(x): fp16(w fp16(x / sqrt(mean(x^2) + eps)))   (norm_weight)
@@ -331,8 +335,8 @@ int aq_qlinear_noalloc(const void* x, int64_t M, int64_t K, int64_t N, const voi
  *             and nothing else folded: the SwiGLU pair, fp16(fp16(silu(g)) u)
  *             written to ys[0] (ys[1] is not written).
  * tile_ptrs, tile_ents: the members' outlier block lists (aq_outlier_tiles)
- * or NULL; at 6 <= M <= 64 the GEMV adds the outliers with MFMAs from them
- * (without them: from the CSR lists, slower).
+ * or NULL; at 6 <= M <= 64 the linears add the outliers with MFMAs from them
+ * (without them, and on tall groups at M > 32: the GEMV, from the CSR lists).
  * relu and residuals may be NULL (none for every member).  The residual
  * must not be the output.  Replaces, at decode, the norm / activation /
  * residual operations of HF's decoder layers around the reference's
@@ -347,10 +351,13 @@ int aq_qlinear_decode(const void* x, int64_t M, int64_t K, int fmt, int64_t coun
 
 /*
  * aq_qlinear_decode with a workspace, as aq_qlinear_grouped's: with
- * aq_qlinear_decode_workspace_size(M, sum of Ns, K) bytes (0 for most calls),
- * calls of 33 to 64 rows with the block lists split K over workgroups and keep
- * the fp32 partial sums there (less: a smaller split; NULL, or too little: the
- * GEMV).
+ * aq_qlinear_decode_workspace_size(M, sum of Ns, K) bytes, calls of 33 to 64
+ * rows with the block lists split K over workgroups and keep the fp32 partial
+ * sums there (less: a smaller split; NULL, or too little: the GEMV).  The size
+ * is 0 for the calls that always take the GEMV: other row counts, short rows
+ * (K < 4096; < 2560 from 49 rows on; < 12288 above 256 tile rows) on grids of
+ * fewer than 384 tile rows, grids of 384 to 1535, and taller ones up to 48 rows
+ * of x or with K < 2048.
  */
 int64_t aq_qlinear_decode_workspace_size(int64_t M, int64_t N, int64_t K);
 int aq_qlinear_decode_ws(const void* x, int64_t M, int64_t K, int fmt, int64_t count, const int64_t* Ns,

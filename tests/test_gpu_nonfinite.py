@@ -1,6 +1,6 @@
 """Infinite and NaN activations through the linear that splits K (33 to 64
-rows): the infinities and NaN of x times the dequantized weight, as F.linear
-gives them, in the outliers' columns and beside them."""
+rows) and the GEMM: the infinities and NaN of x times the dequantized weight, as
+F.linear gives them, in the outliers' columns and beside them."""
 import numpy as np
 import pytest
 import torch
@@ -68,6 +68,14 @@ def test_infinities_stay(N, K, G, fmt, M):
     _check(y, x, deq, bias)
     assert torch.equal(AW.qlinear_decode(x, [q], [bias], [codes], tiles=[tiles])[0].view(torch.int16),
                        y.view(torch.int16))
+
+
+@pytest.mark.parametrize("M", [49, 130])
+@pytest.mark.parametrize("G,fmt", [(-1, "e4m3"), (128, "int8")])
+def test_infinities_stay_in_the_gemm(G, fmt, M):
+    q, deq = _weight(272, 1024, G, fmt, 3)
+    x = _x(M, 1024, deq, q, M)
+    _check(AW.qlinear(x, q, None, codes=AQ.kernel_codes(q, DEV), tiles=AQ.outlier_tiles(q, DEV)), x, deq)
 
 
 def test_infinities_stay_in_groups():
