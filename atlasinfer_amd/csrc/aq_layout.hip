@@ -116,20 +116,22 @@ __device__ __forceinline__ uint64_t load8(const uint8_t* p) {
 }
 __device__ __forceinline__ uint64_t low_bytes(int n) { return ((uint64_t)1 << (8 * n)) - 1; }  // n < 8
 
+// Whether positions c0 .. c0 + 7 lie in a stream of `len` codes (one comparison).
+__device__ __forceinline__ bool in_stream8(int64_t c0, int64_t len) {
+  return (uint64_t)c0 < (uint64_t)max(len - 7, (int64_t)0);
+}
+
 // The codes of a run from a compacted stream of `len` codes: n - popcount(bits)
 // of them from position c0 on, a 0 code put in at each flagged element.
 // Nothing outside the stream is read: c0 is negative after repeated indices.
 __device__ __forceinline__ uint64_t stream_codes(const uint8_t* stream, int64_t len, int64_t c0, uint32_t bits,
                                                  int n) {
   uint64_t w = 0;
-  if (c0 < 0) return w;
-  const uint8_t* src = stream + c0;
-  const int64_t avail = len - c0;
-  if (avail >= 8) {
-    w = load8(src);
-  } else {
+  if (in_stream8(c0, len)) {
+    w = load8(stream + c0);
+  } else if (c0 >= 0) {
     const int need = n - __builtin_popcount(bits);
-    for (int b = 0; b < need && b < avail; b++) w |= (uint64_t)src[b] << (8 * b);
+    for (int b = 0; b < need && c0 + b < len; b++) w |= (uint64_t)stream[c0 + b] << (8 * b);
   }
   while (bits) {
     const int e = __builtin_ctz(bits);
@@ -176,7 +178,8 @@ __global__ __launch_bounds__(256) void reorder_codes_kernel(const uint8_t* src, 
         bits &= (1u << n) - 1u;
       }
       const int left = n - __builtin_popcount(bits);
-      if (c0 < 0 || c0 + left > padded - nnz) continue;  // only after indices that do not ascend
+      // outside the stream only after indices that do not ascend
+      if (!in_stream8(c0, padded - nnz) && (c0 < 0 || c0 + left > padded - nnz)) continue;
       while (bits) {  // from the last flagged element down
         const int e = 31 - __builtin_clz(bits);
         bits &= ~(1u << e);
