@@ -30,6 +30,7 @@
 
 #include "aq_common.h"
 #include "aq_qlinear_internal.h"
+#include "aq_tiles.h"
 
 namespace {
 
@@ -350,24 +351,37 @@ __global__ __launch_bounds__(64 * kMidWaves, 2) void qlinear_mid_kernel(QLArgs a
   }
 }
 
+// The launch's arguments read again from where they lie, so that a rare path's
+// share of them is not loaded, or picked out of the group, before it is taken.
+typedef const __attribute__((address_space(4))) QLArgs* KernelArgs;
+__device__ __forceinline__ KernelArgs kernel_args() {
+  uint64_t p = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();  // QLArgs is the only argument
+  asm volatile("" : "+s"(p));
+  return (KernelArgs)p;
+}
+
+// What mid_infinite reads of a matrix.
+struct MidWeight {
+  const uint8_t* codes;
+  const uint16_t* scales;
+  const int32_t* row_ptr;
+  const int32_t* cols;
+  const uint16_t* vals;
+  int G, kg, gshift;
+};
+
 // The dequantized weight at (n, k): an outlier's value where the code is 0 and
 // the row's list has the column.
 template <int FMT>
-__device__ __forceinline__ float weight_at(const QLMat& w, int K, int n, int k) {
+__device__ __forceinline__ float weight_at(const MidWeight& w, int K, int n, int k) {
   const uint32_t code = w.codes[tiled_offset(n, k, K >> 7)];
   if (code == 0) {
-    int lo = w.row_ptr[n], hi = w.row_ptr[n + 1];
-    const int end = hi;
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if (w.cols[mid] < k)
-        lo = mid + 1;
-      else
-        hi = mid;
-    }
-    if (lo < end && w.cols[lo] == k) return (float)bits_to_h(w.vals[lo]);
+    const int end = w.row_ptr[n + 1];
+    const int p = aq::lower_bound_i32(w.cols, w.row_ptr[n], end, k);
+    if (p < end && w.cols[p] == k) return (float)bits_to_h(w.vals[p]);
   }
-  return (float)deq8<FMT>(code, 0u, scale2(w.scales[scale_index(w, n, k)]))[0];
+  const uint16_t s = w.scales[(size_t)n * w.kg + (w.gshift >= 0 ? k >> w.gshift : k / w.G)];
+  return (float)deq8<FMT>(code, 0u, scale2(s))[0];
 }
 
 __device__ __forceinline__ bool not_finite(uint32_t h) { return (h & 0x7C00u) == 0x7C00u; }
@@ -381,8 +395,12 @@ __device__ __forceinline__ bool not_finite(uint32_t h) { return (h & 0x7C00u) ==
 // (Weights that are not finite themselves: all terms.)  Rows of x with a NaN,
 // or that are finite, keep theirs.  Every lane of the wave calls it.
 template <int FMT>
-__device__ __forceinline__ void mid_infinite(const QLArgs& a, const QLMat& w, int m, int n, bool live, float (&v)[4]) {
-  const int lane = threadIdx.x & 63, K = a.K;
+__device__ __forceinline__ void mid_infinite(int mat, int m, int n, bool live, float (&v)[4]) {
+  const KernelArgs a = kernel_args();
+  const MidWeight w = {a->mat[mat].codes, a->mat[mat].scales, a->mat[mat].row_ptr, a->mat[mat].cols,
+                       a->mat[mat].vals,  a->mat[mat].G,      a->mat[mat].kg,      a->mat[mat].gshift};
+  const int lane = threadIdx.x & 63, K = a->K;
+  const uint16_t* x = a->x;
   const bool nan = live && (v[0] != v[0] || v[1] != v[1] || v[2] != v[2] || v[3] != v[3]);
   uint64_t todo = __ballot(nan);
   while (todo) {
@@ -400,7 +418,7 @@ __device__ __forceinline__ void mid_infinite(const QLArgs& a, const QLMat& w, in
     for (int k0 = 0; k0 < K && !stop; k0 += 512) {
       const int k = k0 + 8 * lane;
       u32x4 xv = (u32x4){0, 0, 0, 0};
-      if (k < K) xv = *reinterpret_cast<const u32x4*>(a.x + (size_t)mr * K + k);
+      if (k < K) xv = *reinterpret_cast<const u32x4*>(x + (size_t)mr * K + k);
       uint32_t take = 0, nans = 0;
 #pragma unroll
       for (int j = 0; j < 8; j++) {
@@ -440,32 +458,48 @@ __device__ __forceinline__ void mid_infinite(const QLArgs& a, const QLMat& w, in
 // thread; grid row y is matrix y (the pair's gate).
 template <int FMT, int PAIR>
 __global__ __launch_bounds__(256) void mid_reduce_kernel(QLArgs a) {
-  const QLMat W = pick(a, (int)blockIdx.y);
+  const QLMat W = PAIR ? a.mat[0] : pick(a, (int)blockIdx.y);
   const int N = W.N;
   const int64_t mn = (int64_t)a.M * N;
   const int64_t i0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
   const bool live = i0 < mn;
   const int64_t i = live ? i0 : 0;
   const int m = (int)(i / N), n = (int)(i - (int64_t)m * N);  // N is a multiple of 16: the 4 columns are of one row
-  auto sum = [&](const QLMat& w, float (&v)[4]) {
+  // every load goes out before the sums are looked at
+  auto sum = [&](const QLMat& w, float (&v)[4], float (&bias)[4]) {
     float4v s = *reinterpret_cast<const float4v*>(w.part + i);
     for (int p = 1; p < a.split; p++) s += *reinterpret_cast<const float4v*>(w.part + (size_t)p * mn + i);
 #pragma unroll
-    for (int j = 0; j < 4; j++) v[j] = s[j];
-    const bool nan = v[0] != v[0] || v[1] != v[1] || v[2] != v[2] || v[3] != v[3];
-    if (__builtin_expect(__ballot(live && nan) != 0, 0)) mid_infinite<FMT>(a, w, m, n, live, v);
-#pragma unroll
-    for (int j = 0; j < 4; j++) v[j] += w.bias ? (float)bits_to_h(w.bias[n + j]) : 0.0f;
+    for (int j = 0; j < 4; j++) {
+      v[j] = s[j];
+      bias[j] = w.bias ? (float)bits_to_h(w.bias[n + j]) : 0.0f;
+    }
   };
-  float v[4], u[4];
-  sum(W, v);
-  if (PAIR) sum(a.mat[1], u);
+  float v[4], u[4], bv[4], bu[4];
+  uint16_t res[4] = {0, 0, 0, 0};
+  sum(W, v, bv);
+  if (PAIR) sum(a.mat[1], u, bu);
+  if (!PAIR && W.res)
+#pragma unroll
+    for (int j = 0; j < 4; j++) res[j] = W.res[i + j];
+  bool nan = false;
+#pragma unroll
+  for (int j = 0; j < 4; j++) nan = nan || v[j] != v[j] || (PAIR && u[j] != u[j]);
+  if (__builtin_expect(__ballot(live && nan) != 0, 0)) {
+    mid_infinite<FMT>((int)blockIdx.y, m, n, live, v);
+    if (PAIR) mid_infinite<FMT>(1, m, n, live, u);
+  }
   if (!live) return;
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    v[j] += bv[j];
+    if (PAIR) u[j] += bu[j];
+  }
   uint16_t o[4];
 #pragma unroll
   for (int j = 0; j < 4; j++)
     o[j] = PAIR ? h_to_bits(silu_mul_h((float)rn_h(v[j]), (float)rn_h(u[j])))
-                : mid_epilogue(rn_h(v[j]), W.act, W.res ? W.res[i + j] : (uint16_t)0, W.res != nullptr);
+                : mid_epilogue(rn_h(v[j]), W.act, res[j], W.res != nullptr);
   if ((uintptr_t)W.y % 8 == 0) {
     *reinterpret_cast<uint2*>(W.y + i) = make_uint2(o[0] | ((uint32_t)o[1] << 16), o[2] | ((uint32_t)o[3] << 16));
   } else {
